@@ -25,6 +25,9 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
+#include <utility>
 #include <vector>
 
 using namespace mdx;
@@ -57,6 +60,23 @@ namespace {
 struct Buf {
     void *p = nullptr;
     size_t bytes = 0;
+};
+
+// device-to-host copies (fetch): up to FETCH_THREADS host threads, each with
+// two pinned slots of at most FETCH_CHUNK bytes
+constexpr int FETCH_THREADS = 4;
+constexpr size_t FETCH_CHUNK = (size_t)4 << 20;
+constexpr size_t FETCH_SMALL = (size_t)2 << 20; // one slot, one thread, up to here
+// host-to-device copies through the pinned slot up to here (64 KB: 10 us
+// against 32 us pageable; from 128 KB on the two are equal)
+constexpr size_t UPLOAD_PINNED = (size_t)128 << 10;
+constexpr size_t FETCH_CHUNK_MIN = (size_t)256 << 10;
+
+// one host array and the device array it is filled from
+struct Span {
+    void *host;
+    const void *dev;
+    size_t bytes;
 };
 
 struct GraphSlot {
@@ -135,6 +155,13 @@ struct mdx_engine {
     Buf ang_off, ang_ref, ang_ijk, ang_k, ang_t0;
     Buf exc_off, exc_j, act_prev, act_next;
     Buf noise, ctl, partial, tmpd, tmpi, tmpi2, tmpi3, tmpll, tmpx;
+    // pinned staging of the device-to-host copies (fetch): at most
+    // 2 FETCH_THREADS FETCH_CHUNK = 32 MiB, given back with the engine
+    char *pin = nullptr;
+    size_t pin_bytes = 0;
+    hipEvent_t pin_ev[2 * FETCH_THREADS] = {};
+    Buf dmeta; // meta by original index (uploaded when it changed)
+    bool meta_dirty = true;
     Buf Fw, ncand, cand, Tp; // split walk -> (patch ->) finish
     int use_compact = 1;     // compacted patch kernel + integrate kernel (MDX_COMPACT=0: one finish kernel)
     int use_walkc = 1;       // compacted list walk (MDX_WALKC=0: one lane per position)
@@ -192,23 +219,207 @@ static void dfree(Buf &b)
     b.bytes = 0;
 }
 
+// Pinned host memory of destroyed (or grown) engines, for the next engine that
+// needs some: pinning costs 0.05 to 0.3 ms a time, as much as creating a small
+// engine.  At most PIN_POOL bytes in PIN_POOL_N pieces are held, under a lock; a buffer belongs to
+// one engine while that engine holds it.
+constexpr size_t PIN_POOL = (size_t)64 << 20;
+constexpr int PIN_POOL_N = 16;
+static std::mutex g_pin_mu;
+static std::pair<char *, size_t> g_pin_free[PIN_POOL_N];
+static int g_pin_count = 0;
+static size_t g_pin_held = 0;
+
+static void pin_release(mdx_engine *e)
+{
+    if (!e->pin)
+        return;
+    {
+        std::lock_guard<std::mutex> lock(g_pin_mu);
+        if (g_pin_count < PIN_POOL_N && g_pin_held + e->pin_bytes <= PIN_POOL) {
+            g_pin_free[g_pin_count++] = {e->pin, e->pin_bytes};
+            g_pin_held += e->pin_bytes;
+            e->pin = nullptr;
+        }
+    }
+    if (e->pin)
+        (void)hipHostFree(e->pin);
+    e->pin = nullptr;
+    e->pin_bytes = 0;
+}
+
+// (only between the copies of one call: nothing in flight uses the old one)
+static int pin_reserve(mdx_engine *e, size_t bytes)
+{
+    if (e->pin_bytes >= bytes)
+        return MDX_OK;
+    pin_release(e);
+    {
+        // the smallest that fits, unless it is far too large
+        std::lock_guard<std::mutex> lock(g_pin_mu);
+        int at = -1;
+        for (int k = 0; k < g_pin_count; k++)
+            if (g_pin_free[k].second >= bytes && g_pin_free[k].second <= 8 * bytes &&
+                (at < 0 || g_pin_free[k].second < g_pin_free[at].second))
+                at = k;
+        if (at >= 0) {
+            e->pin = g_pin_free[at].first;
+            e->pin_bytes = g_pin_free[at].second;
+            g_pin_held -= e->pin_bytes;
+            g_pin_free[at] = g_pin_free[--g_pin_count];
+            return MDX_OK;
+        }
+    }
+    HIPCHK(hipHostMalloc((void **)&e->pin, bytes, hipHostMallocPortable));
+    e->pin_bytes = bytes;
+    return MDX_OK;
+}
+
+// one slot of at least the given size (at most FETCH_SMALL), a power of two
+// that holds a small engine's whole state
+static int pin_small(mdx_engine *e, size_t bytes)
+{
+    size_t need = (size_t)64 << 10;
+    while (need < std::max(bytes, std::min(FETCH_SMALL, 144 * (size_t)e->N)))
+        need *= 2;
+    return pin_reserve(e, need);
+}
+
 template <class T> static int upload(mdx_engine *e, Buf &b, const T *h, size_t n)
 {
     int rc = dalloc(e, b, n * sizeof(T));
     if (rc)
         return rc;
+    const void *src = h;
+    if (n && n * sizeof(T) <= UPLOAD_PINNED) {
+        if ((rc = pin_small(e, n * sizeof(T))))
+            return rc;
+        std::memcpy(e->pin, h, n * sizeof(T));
+        src = e->pin;
+    }
     if (n)
-        HIPCHK(hipMemcpyAsync(b.p, h, n * sizeof(T), hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(b.p, src, n * sizeof(T), hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
+    return MDX_OK;
+}
+
+// Device arrays into the caller's (pageable, often never touched) arrays,
+// complete on return.  A pageable device-to-host copy runs at 18 GB/s into
+// touched memory and at half of that into fresh pages, one thread faulting
+// them; the link carries 57 GB/s.  So the copies go through pinned slots and
+// the host threads that empty them fault and fill the caller's pages in
+// parallel: 151 MB into fresh pages took 14.8 ms as one pageable copy, and
+// through the slots 11.3 ms with 1 thread, 6.2 with 2, 4.0 with 4, 3.8 with
+// 8.  Up to FETCH_SMALL bytes one slot, no threads and no events, and one copy
+// where the caller says that the device arrays follow each other in one
+// allocation: a pageable copy costs 7 to 20 us of its own (64 KB: 34 us
+// against 10, 600 KB in two arrays: 39 against 32).
+static int fetch(mdx_engine *e, const Span *sp, int n, bool joined = false)
+{
+    size_t total = 0;
+    for (int k = 0; k < n; k++)
+        total += sp[k].bytes;
+    if (total == 0) {
+        HIPCHK(hipStreamSynchronize(e->stream));
+        return MDX_OK;
+    }
+    int rc;
+    if (total <= FETCH_SMALL) {
+        if ((rc = pin_small(e, total)))
+            return rc;
+        size_t off = 0;
+        for (int k = 0; k < (joined ? 1 : n); k++) {
+            const size_t len = joined ? total : sp[k].bytes;
+            if (len)
+                HIPCHK(hipMemcpyAsync(e->pin + off, sp[k].dev, len, hipMemcpyDeviceToHost,
+                                      e->stream));
+            off += len;
+        }
+        HIPCHK(hipStreamSynchronize(e->stream));
+        off = 0;
+        for (int k = 0; k < n; k++) {
+            if (sp[k].bytes)
+                std::memcpy(sp[k].host, e->pin + off, sp[k].bytes);
+            off += sp[k].bytes;
+        }
+        return MDX_OK;
+    }
+    // slots sized so that every thread has a few
+    const int T = total < 4 * FETCH_SMALL ? 2 : FETCH_THREADS;
+    const size_t C =
+        std::min(FETCH_CHUNK, std::max(FETCH_CHUNK_MIN, (total / (4 * T) + 4095) & ~(size_t)4095));
+    if ((rc = pin_reserve(e, 2 * T * C)))
+        return rc;
+    for (int k = 0; k < 2 * T; k++)
+        if (!e->pin_ev[k])
+            HIPCHK(hipEventCreateWithFlags(&e->pin_ev[k], hipEventDisableTiming));
+    // piece c of all spans, C bytes at a time (a piece ends with its span)
+    size_t pieces = 0;
+    for (int k = 0; k < n; k++)
+        pieces += (sp[k].bytes + C - 1) / C;
+    auto piece = [&](size_t c, char *&h, const char *&d, size_t &len) {
+        int k = 0;
+        for (; c >= (sp[k].bytes + C - 1) / C; k++)
+            c -= (sp[k].bytes + C - 1) / C;
+        h = (char *)sp[k].host + c * C;
+        d = (const char *)sp[k].dev + c * C;
+        len = std::min(C, sp[k].bytes - c * C);
+    };
+    hipError_t err[FETCH_THREADS] = {};
+    // thread k: pieces k, k + T, ...; its two slots in turn
+    auto work = [&](int k) {
+        hipError_t he = hipSetDevice(e->device);
+        char *h;
+        const char *d;
+        size_t len;
+        auto issue = [&](size_t c, int s) {
+            piece(c, h, d, len);
+            if (he == hipSuccess)
+                he = hipMemcpyAsync(e->pin + (2 * k + s) * C, d, len, hipMemcpyDeviceToHost, e->stream);
+            if (he == hipSuccess)
+                he = hipEventRecord(e->pin_ev[2 * k + s], e->stream);
+        };
+        int s = 0;
+        if ((size_t)k < pieces)
+            issue(k, 0);
+        for (size_t c = k; c < pieces && he == hipSuccess; c += T, s ^= 1) {
+            if (c + T < pieces)
+                issue(c + T, s ^ 1);
+            if (he == hipSuccess)
+                he = hipEventSynchronize(e->pin_ev[2 * k + s]);
+            if (he == hipSuccess) {
+                piece(c, h, d, len);
+                std::memcpy(h, e->pin + (2 * k + s) * C, len);
+            }
+        }
+        err[k] = he;
+    };
+    std::thread th[FETCH_THREADS];
+    bool own[FETCH_THREADS] = {};
+    for (int k = 1; k < T; k++) {
+        try {
+            th[k] = std::thread(work, k);
+        } catch (const std::system_error &) {
+            own[k] = true; // no thread to be had: its pieces are done here
+        }
+    }
+    work(0);
+    for (int k = 1; k < T; k++) {
+        if (own[k])
+            work(k);
+        else
+            th[k].join();
+    }
+    HIPCHK(hipStreamSynchronize(e->stream));
+    for (int k = 0; k < T; k++)
+        HIPCHK(err[k]);
     return MDX_OK;
 }
 
 template <class T> static int download(mdx_engine *e, const Buf &b, T *h, size_t n)
 {
-    if (n)
-        HIPCHK(hipMemcpyAsync(h, b.p, n * sizeof(T), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
-    return MDX_OK;
+    const Span sp = {h, b.p, n * sizeof(T)};
+    return fetch(e, &sp, 1);
 }
 
 static inline unsigned nblk(long long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
@@ -592,8 +803,9 @@ static int launch_gather(mdx_engine *e, const double *noise_dev, int lmode = 0)
 static int read_status(mdx_engine *e, unsigned int *st, long long *step = nullptr)
 {
     StepCtl c;
-    HIPCHK(hipMemcpyAsync(&c, e->ctl.p, sizeof c, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    int rc;
+    if ((rc = download(e, e->ctl, &c, 1)))
+        return rc;
     *st = c.status;
     if (step)
         *step = c.status ? (long long)(c.fail_epoch - c.call_base) : -1;
@@ -985,45 +1197,15 @@ static int slot_ids(mdx_engine *e, std::vector<PosRec> &rec)
     return download(e, e->X[e->cur], rec.data(), rec.size());
 }
 
-template <class R> static int upload_real(mdx_engine *e, Buf &dst, const double *h, size_t n)
+// meta by original index on the device
+static int meta_upload(mdx_engine *e)
 {
-    if (sizeof(R) == 8)
-        return upload(e, dst, h, n);
-    int rc = upload(e, e->tmpd, h, n);
-    if (rc)
-        return rc;
-    hipLaunchKernelGGL((k_convert<double, R>), dim3(nblk((long long)n)), dim3(256), 0, e->stream,
-                       (const double *)e->tmpd.p, (R *)dst.p, n);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(e->stream));
-    return MDX_OK;
-}
-
-// slot-ordered device array (width values per particle) to a host array in
-// original order
-template <class R>
-static int download_by_id(mdx_engine *e, const Buf &src, const std::vector<PosRec> &rec, int width,
-                          double *h)
-{
-    const size_t n = (size_t)e->N * width;
-    std::vector<double> tmp(n);
-    if (sizeof(R) == 8) {
-        int rc = download(e, src, tmp.data(), n);
-        if (rc)
-            return rc;
-    } else {
-        int rc = dalloc(e, e->tmpd, n * 8);
-        if (rc)
-            return rc;
-        hipLaunchKernelGGL((k_convert<R, double>), dim3(nblk((long long)n)), dim3(256), 0,
-                           e->stream, (const R *)src.p, (double *)e->tmpd.p, n);
-        HIPCHK(hipGetLastError());
-        if ((rc = download(e, e->tmpd, tmp.data(), n)))
-            return rc;
-    }
-    for (int s = 0; s < e->N; s++)
-        std::memcpy(h + (size_t)rec[s].id * width, tmp.data() + (size_t)s * width, 8 * width);
-    return MDX_OK;
+    if (!e->meta_dirty)
+        return MDX_OK;
+    int rc = upload(e, e->dmeta, e->meta.data(), e->meta.size());
+    if (!rc)
+        e->meta_dirty = false;
+    return rc;
 }
 
 // ================================================================== C ABI
@@ -1174,9 +1356,13 @@ void mdx_destroy(mdx_engine *e)
                    &e->dslot,   &e->Tp,      &e->bpoff,  &e->bowner, &e->bisbound, &e->bboundto,
                    &e->badj_n,  &e->badj_p,  &e->badj_s, &e->bF,     &e->bT,      &e->bscr,
                    &e->bnscr,   &e->bspecies, &e->bdtab, &e->bttab,  &e->btr4,
-                   &e->plpairs, &e->plmask};
+                   &e->plpairs, &e->plmask, &e->dmeta};
     for (Buf *b : bufs)
         dfree(*b);
+    for (hipEvent_t ev : e->pin_ev)
+        if (ev)
+            (void)hipEventDestroy(ev);
+    pin_release(e);
     for (GraphSlot &g : e->graphs)
         if (g.exec)
             (void)hipGraphExecDestroy(g.exec);
@@ -1200,48 +1386,46 @@ static int upload_state_t(mdx_engine *e, const double *x, const double *p, const
                           const double *L)
 {
     const size_t N = e->N;
-    e->cur = 0;
-    std::vector<PosRec> rec(N);
-    std::vector<int> slot(N);
-    for (size_t i = 0; i < N; i++) {
-        rec[i].x = x[3 * i];
-        rec[i].y = x[3 * i + 1];
-        rec[i].z = x[3 * i + 2];
-        rec[i].id = (uint32_t)i;
-        rec[i].meta = e->meta[i];
-        slot[i] = (int)i;
-    }
+    const bool rot = e->integ == MDX_INTEG_ROTOR;
+    // the caller's arrays back to back in tmpd (18 doubles per particle at
+    // most), checked there; the state is written only if all are finite
     int rc;
-    if ((rc = upload(e, e->X[0], rec.data(), N)) || (rc = upload(e, e->slot[0], slot.data(), N)))
+    if ((rc = dalloc(e, e->tmpd, 8 * 18 * N)) || (rc = dalloc(e, e->tmpll, 2 * sizeof(unsigned int))) ||
+        (rc = meta_upload(e)))
         return rc;
-    std::vector<double> z;
-    if (!p || (!L && e->integ == MDX_INTEG_ROTOR))
-        z.assign(3 * N, 0.0);
-    if ((rc = upload_real<R>(e, e->P[0], p ? p : z.data(), 3 * N)))
-        return rc;
-    if (e->integ == MDX_INTEG_ROTOR) {
-        if ((rc = upload_real<R>(e, e->Lm[0], L ? L : z.data(), 3 * N)))
-            return rc;
-        std::vector<double> eye;
-        if (!Q) {
-            eye.assign(9 * N, 0.0);
-            for (size_t i = 0; i < N; i++)
-                eye[9 * i] = eye[9 * i + 4] = eye[9 * i + 8] = 1.0;
-        }
-        const double *Qh = Q ? Q : eye.data();
-        if (sizeof(R) == 8) {
-            if ((rc = upload(e, e->Q[0], Qh, 9 * N)))
-                return rc;
-        } else {
-            // the mixed engine stores unit quaternions
-            if ((rc = upload(e, e->tmpd, Qh, 9 * N)))
-                return rc;
-            hipLaunchKernelGGL(k_mats_to_quats, dim3(nblk((long long)N)), dim3(256), 0, e->stream,
-                               (const double *)e->tmpd.p, (int)N, (float *)e->Q[0].p);
-            HIPCHK(hipGetLastError());
-            HIPCHK(hipStreamSynchronize(e->stream));
-        }
+    const double *const src[4] = {x, p, L, Q};
+    const int width[4] = {3, 3, 3, 9};
+    const double *dev[4];
+    double *at = (double *)e->tmpd.p;
+    for (int k = 0; k < 4; k++) {
+        dev[k] = src[k] ? at : nullptr;
+        if (!src[k])
+            continue;
+        HIPCHK(hipMemcpyAsync(at, src[k], 8 * width[k] * N, hipMemcpyHostToDevice, e->stream));
+        at += width[k] * N;
     }
+    unsigned int *bad = (unsigned int *)e->tmpll.p; // first bad particle: momenta, orientations
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, e->stream, bad, 2, ~0u);
+    hipLaunchKernelGGL(k_check_state, dim3(nblk((long long)N)), dim3(256), 0, e->stream, (int)N,
+                       dev[0], dev[1], dev[2], dev[3], bad);
+    hipLaunchKernelGGL(k_state_from_host<R>, dim3(nblk((long long)N)), dim3(256), 0, e->stream,
+                       (int)N, dev[0], dev[1], rot ? dev[2] : nullptr, rot ? dev[3] : nullptr,
+                       (const uint32_t *)e->dmeta.p, (const unsigned int *)bad, (PosRec *)e->X[0].p,
+                       (R *)e->P[0].p, rot ? (R *)e->Lm[0].p : nullptr,
+                       rot ? (R *)e->Q[0].p : nullptr, (int *)e->slot[0].p);
+    HIPCHK(hipGetLastError());
+    unsigned int first[2];
+    if ((rc = download(e, e->tmpll, first, 2)))
+        return rc;
+    if (first[0] != ~0u)
+        return set_err(MDX_ERR_ARG, "non-finite position or momentum at particle %u", first[0]);
+    if (first[1] != ~0u)
+        return set_err(MDX_ERR_ARG, "non-finite orientation at particle %u", first[1]);
+    e->cur = 0;
+    e->binned = false;
+    e->primed = false;
+    e->counted = false;
+    e->list_valid = false;
     return MDX_OK;
 }
 
@@ -1251,20 +1435,44 @@ int mdx_upload_state(mdx_engine *e, const double *x, const double *p, const doub
     if (!e || !x)
         return set_err(MDX_ERR_ARG, "engine and positions required");
     HIPCHK(hipSetDevice(e->device));
-    for (long long k = 0; k < 3ll * e->N; k++)
-        if (!std::isfinite(x[k]) || (p && !std::isfinite(p[k])) || (L && !std::isfinite(L[k])))
-            return set_err(MDX_ERR_ARG, "non-finite position or momentum at particle %lld", k / 3);
-    if (Q)
-        for (long long k = 0; k < 9ll * e->N; k++)
-            if (!std::isfinite(Q[k]))
-                return set_err(MDX_ERR_ARG, "non-finite orientation at particle %lld", k / 9);
-    int rc = e->prec == MDX_PREC_FP64 ? upload_state_t<double>(e, x, p, Q, L)
-                                      : upload_state_t<float>(e, x, p, Q, L);
-    e->binned = false;
-    e->primed = false;
-    e->counted = false;
-    e->list_valid = false;
-    return rc;
+    return e->prec == MDX_PREC_FP64 ? upload_state_t<double>(e, x, p, Q, L)
+                                    : upload_state_t<float>(e, x, p, Q, L);
+}
+
+// the current state as the caller's arrays: one kernel writes the asked
+// fields by original index in FP64 (k_state_by_id), one pass copies them
+template <class R>
+static int download_state_t(mdx_engine *e, double *x, double *p, double *Q, double *L)
+{
+    const size_t N = e->N;
+    const bool rot = e->integ == MDX_INTEG_ROTOR;
+    const int c = e->cur;
+    double *const dst[4] = {x, p, Q, L};
+    const int width[4] = {3, 3, 9, 3};
+    double *dev[4];
+    Span sp[4];
+    int n = 0, rc;
+    size_t words = 0;
+    for (int k = 0; k < 4; k++)
+        words += dst[k] ? width[k] * N : 0;
+    if (words == 0)
+        return MDX_OK;
+    if ((rc = dalloc(e, e->tmpd, 8 * words)))
+        return rc;
+    double *at = (double *)e->tmpd.p;
+    for (int k = 0; k < 4; k++) {
+        dev[k] = dst[k] ? at : nullptr;
+        if (!dst[k])
+            continue;
+        sp[n++] = {dst[k], at, 8 * width[k] * N};
+        at += width[k] * N;
+    }
+    hipLaunchKernelGGL(k_state_by_id<R>, dim3(nblk((long long)N)), dim3(256), 0, e->stream, (int)N,
+                       (const PosRec *)e->X[c].p, (const R *)e->P[c].p,
+                       rot ? (const R *)e->Q[c].p : nullptr, rot ? (const R *)e->Lm[c].p : nullptr,
+                       dev[0], dev[1], dev[2], dev[3]);
+    HIPCHK(hipGetLastError());
+    return fetch(e, sp, n, true);
 }
 
 int mdx_download_state(mdx_engine *e, double *x, double *p, double *Q, double *L)
@@ -1272,54 +1480,26 @@ int mdx_download_state(mdx_engine *e, double *x, double *p, double *Q, double *L
     if (!e)
         return set_err(MDX_ERR_ARG, "null engine");
     HIPCHK(hipSetDevice(e->device));
-    std::vector<PosRec> rec;
-    int rc = slot_ids(e, rec);
-    if (rc)
+    return e->prec == MDX_PREC_FP64 ? download_state_t<double>(e, x, p, Q, L)
+                                    : download_state_t<float>(e, x, p, Q, L);
+}
+
+// slot-ordered rows of 3 (a, b) as the caller's arrays by original index
+template <class R>
+static int download_rows_t(mdx_engine *e, const Buf &a, const Buf &b, double *A, double *B)
+{
+    const size_t N = e->N;
+    int rc;
+    if ((rc = dalloc(e, e->tmpd, 8 * 6 * N)))
         return rc;
-    if (x)
-        for (int s = 0; s < e->N; s++) {
-            double *o = x + 3 * (size_t)rec[s].id;
-            o[0] = rec[s].x;
-            o[1] = rec[s].y;
-            o[2] = rec[s].z;
-        }
-    const bool f64 = e->prec == MDX_PREC_FP64;
-    const bool rot = e->integ == MDX_INTEG_ROTOR;
-    const int c = e->cur;
-    if (p && (rc = f64 ? download_by_id<double>(e, e->P[c], rec, 3, p)
-                       : download_by_id<float>(e, e->P[c], rec, 3, p)))
-        return rc;
-    if (Q) {
-        if (rot) {
-            if (f64) {
-                if ((rc = download_by_id<double>(e, e->Q[c], rec, 9, Q)))
-                    return rc;
-            } else {
-                // quaternions as FP64 matrices, then by original index
-                if ((rc = dalloc(e, e->tmpx, 72 * (size_t)e->N)))
-                    return rc;
-                hipLaunchKernelGGL(k_quats_to_mats, dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                                   (const float *)e->Q[c].p, e->N, (double *)e->tmpx.p);
-                HIPCHK(hipGetLastError());
-                if ((rc = download_by_id<double>(e, e->tmpx, rec, 9, Q)))
-                    return rc;
-            }
-        } else {
-            for (int i = 0; i < e->N; i++)
-                for (int k = 0; k < 9; k++)
-                    Q[9 * (size_t)i + k] = (k % 4 == 0) ? 1.0 : 0.0;
-        }
-    }
-    if (L) {
-        if (rot) {
-            if ((rc = f64 ? download_by_id<double>(e, e->Lm[c], rec, 3, L)
-                          : download_by_id<float>(e, e->Lm[c], rec, 3, L)))
-                return rc;
-        } else {
-            std::fill(L, L + 3 * (size_t)e->N, 0.0);
-        }
-    }
-    return MDX_OK;
+    double *da = A ? (double *)e->tmpd.p : nullptr;
+    double *db = B ? (double *)e->tmpd.p + 3 * N : nullptr;
+    hipLaunchKernelGGL(k_state_by_id<R>, dim3(nblk((long long)N)), dim3(256), 0, e->stream, (int)N,
+                       (const PosRec *)e->X[e->cur].p, (const R *)a.p, (const R *)nullptr,
+                       (const R *)b.p, (double *)nullptr, da, (double *)nullptr, db);
+    HIPCHK(hipGetLastError());
+    const Span sp[2] = {{A, da, A ? 24 * N : 0}, {B, db, B ? 24 * N : 0}};
+    return fetch(e, sp, 2);
 }
 
 int mdx_download_forces(mdx_engine *e, double *F, double *T)
@@ -1329,19 +1509,9 @@ int mdx_download_forces(mdx_engine *e, double *F, double *T)
     if (!e->primed || e->integ != MDX_INTEG_ROTOR)
         return set_err(MDX_ERR_STATE, "no carried forces (rotor engine: prime or step first)");
     HIPCHK(hipSetDevice(e->device));
-    std::vector<PosRec> rec;
-    int rc = slot_ids(e, rec);
-    if (rc)
-        return rc;
-    const bool f64 = e->prec == MDX_PREC_FP64;
     const int c = e->cur;
-    if (F && (rc = f64 ? download_by_id<double>(e, e->Fc[c], rec, 3, F)
-                       : download_by_id<float>(e, e->Fc[c], rec, 3, F)))
-        return rc;
-    if (T && (rc = f64 ? download_by_id<double>(e, e->Tc[c], rec, 3, T)
-                       : download_by_id<float>(e, e->Tc[c], rec, 3, T)))
-        return rc;
-    return MDX_OK;
+    return e->prec == MDX_PREC_FP64 ? download_rows_t<double>(e, e->Fc[c], e->Tc[c], F, T)
+                                    : download_rows_t<float>(e, e->Fc[c], e->Tc[c], F, T);
 }
 
 int mdx_set_pair_wca(mdx_engine *e, double eps, double sigma, double rcut)
@@ -1447,10 +1617,11 @@ int mdx_set_patches(mdx_engine *e, int ntypes, const int *type_of_particle,
             e->meta[i] = ((uint32_t)r << 8) | (uint32_t)type_of_particle[i];
         }
     int rc;
-    if ((rc = upload(e, e->tmpi, e->meta.data(), e->meta.size())))
+    e->meta_dirty = true;
+    if ((rc = meta_upload(e)))
         return rc;
     hipLaunchKernelGGL(k_set_meta, dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                       (PosRec *)e->X[e->cur].p, e->N, (const uint32_t *)e->tmpi.p);
+                       (PosRec *)e->X[e->cur].p, e->N, (const uint32_t *)e->dmeta.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
     std::vector<double> pd = e->pdirs;
@@ -1942,9 +2113,8 @@ template <class R> static int compute_forces_t(mdx_engine *e, double *F, double 
         return rc;
     if ((rc = launch_gather<R, M_CONS>(e, nullptr)))
         return rc;
-    if ((rc = download(e, e->Fout, F, 3 * (size_t)e->N)))
-        return rc;
-    if (T && (rc = download(e, e->Tout, T, 3 * (size_t)e->N)))
+    const Span out[2] = {{F, e->Fout.p, 24 * (size_t)e->N}, {T, e->Tout.p, T ? 24 * (size_t)e->N : 0}};
+    if ((rc = fetch(e, out, 2)))
         return rc;
     if (e->bind_on) {
         // with binding: the bound pairs' terms of the current bound state
@@ -2700,12 +2870,32 @@ static void stage_done(mdx_engine *e, bool moved)
     }
 }
 
-static int stage_upload(mdx_engine *e, Buf &b, const double *h, size_t n)
+// up to three host arrays (n[k] doubles) into device buffers: through the
+// pinned slot while they fit it (a pageable copy of 64 KB costs 32 us, 10
+// this way), which every single-stage call leaves idle when it returns
+static int stage_upload(mdx_engine *e, int count, Buf *const b[], const double *const h[],
+                        const size_t n[])
 {
-    int rc = dalloc(e, b, n * sizeof(double));
-    if (rc)
+    size_t total = 0, off = 0;
+    int rc;
+    for (int k = 0; k < count; k++) {
+        if ((rc = dalloc(e, *b[k], n[k] * sizeof(double))))
+            return rc;
+        total += n[k] * sizeof(double);
+    }
+    const bool pinned = total <= FETCH_SMALL;
+    if (pinned && (rc = pin_small(e, total)))
         return rc;
-    HIPCHK(hipMemcpyAsync(b.p, h, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
+    for (int k = 0; k < count; k++) {
+        const size_t len = n[k] * sizeof(double);
+        const void *src = h[k];
+        if (pinned) {
+            std::memcpy(e->pin + off, h[k], len);
+            src = e->pin + off;
+            off += len;
+        }
+        HIPCHK(hipMemcpyAsync(b[k]->p, src, len, hipMemcpyHostToDevice, e->stream));
+    }
     return MDX_OK;
 }
 
@@ -2713,10 +2903,11 @@ template <class R> static int stage_halfkick_t(mdx_engine *e, const double *F, c
 {
     int rc;
     const size_t n3 = 3 * (size_t)e->N;
-    if ((rc = stage_upload(e, e->tmpd, F, n3)))
-        return rc;
     const bool rot = e->integ == MDX_INTEG_ROTOR;
-    if (rot && (rc = stage_upload(e, e->tmpx, T, n3)))
+    Buf *const b[] = {&e->tmpd, &e->tmpx};
+    const double *const h[] = {F, T};
+    const size_t n[] = {n3, n3};
+    if ((rc = stage_upload(e, rot ? 2 : 1, b, h, n)))
         return rc;
     hipLaunchKernelGGL(k_stage_halfkick<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, e->N,
                        (const PosRec *)e->X[e->cur].p, (R *)e->P[e->cur].p,
@@ -2787,8 +2978,10 @@ template <class R> static int stage_sphere_t(mdx_engine *e, double *F, double *T
     if (rc)
         return rc;
     const size_t n3 = 3 * (size_t)e->N;
-    if ((rc = stage_upload(e, e->tmpd, F, n3)) || (rc = stage_upload(e, e->tmpx, T, n3)) ||
-        (rc = stage_upload(e, e->noise, RT, 2 * n3)))
+    Buf *const b[] = {&e->tmpd, &e->tmpx, &e->noise};
+    const double *const h[] = {F, T, RT};
+    const size_t n[] = {n3, n3, 2 * n3};
+    if ((rc = stage_upload(e, 3, b, h, n)))
         return rc;
     hipLaunchKernelGGL(k_stage_sphere<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, e->N,
                        (const PosRec *)e->X[e->cur].p, (const R *)e->P[e->cur].p,
@@ -2797,7 +2990,8 @@ template <class R> static int stage_sphere_t(mdx_engine *e, double *F, double *T
                        (const double *)e->noise.p, -e->gamma / e->m, -e->gammar / e->I[0],
                        -e->gammar / e->I[1], -e->gammar / e->I[2]);
     HIPCHK(hipGetLastError());
-    if ((rc = download(e, e->tmpd, F, n3)) || (rc = download(e, e->tmpx, T, n3)))
+    const Span out[2] = {{F, e->tmpd.p, 8 * n3}, {T, e->tmpx.p, 8 * n3}};
+    if ((rc = fetch(e, out, 2)))
         return rc;
     stage_done(e, false);
     return MDX_OK;
@@ -2820,7 +3014,10 @@ template <class R> static int stage_advance_mom_t(mdx_engine *e, const double *F
     if (rc)
         return rc;
     const size_t n3 = 3 * (size_t)e->N;
-    if ((rc = stage_upload(e, e->tmpd, F, n3)) || (rc = stage_upload(e, e->tmpx, Rn, n3)))
+    Buf *const b[] = {&e->tmpd, &e->tmpx};
+    const double *const h[] = {F, Rn};
+    const size_t n[] = {n3, n3};
+    if ((rc = stage_upload(e, 2, b, h, n)))
         return rc;
     const double d = (e->gamma * e->dt / 2.), q = (e->dt) / 2.;
     const double c2 = (1.0 / (1.0 + (d))), c3 = (1.0 / (1.0 + (d))) * q, c5 = (1 - (d));

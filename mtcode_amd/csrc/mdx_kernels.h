@@ -3050,12 +3050,125 @@ __global__ void __launch_bounds__(256) k_sum_rows(int first, int count, const do
     }
 }
 
-// precision conversion (device <-> host FP64 layout)
-template <class A, class B> __global__ void k_convert(const A *in, B *out, size_t n)
+__global__ void k_fill_u32(unsigned int *p, int n, unsigned int v)
 {
-    size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n)
-        out[k] = (B)in[k];
+    for (int k = threadIdx.x; k < n; k += blockDim.x)
+        p[k] = v;
+}
+
+// the first particle with a non-finite position or momentum (bad[0]) and with
+// a non-finite orientation (bad[1]) of an upload, by original index; null
+// arrays are not looked at
+__global__ void k_check_state(int N, const double *x, const double *p, const double *L,
+                              const double *Q, unsigned int *bad)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N)
+        return;
+    bool ok = true, okq = true;
+    for (int k = 0; k < 3; k++) {
+        ok = ok && isfinite(x[3 * (size_t)i + k]);
+        ok = ok && (!p || isfinite(p[3 * (size_t)i + k]));
+        ok = ok && (!L || isfinite(L[3 * (size_t)i + k]));
+    }
+    if (Q)
+        for (int k = 0; k < 9; k++)
+            okq = okq && isfinite(Q[9 * (size_t)i + k]);
+    if (!ok)
+        atomicMin(&bad[0], (unsigned int)i);
+    if (!okq)
+        atomicMin(&bad[1], (unsigned int)i);
+}
+
+// an upload's arrays (FP64, original order) as the state of slots 0..N-1;
+// null p, L: zero, null Q: the identity.  Nothing is written after a failed
+// check.  Mixed: matrices to unit quaternions by Shepperd's method in FP64,
+// rounded once.
+template <class R>
+__global__ void __launch_bounds__(256) k_state_from_host(int N, const double *x, const double *p,
+                                                         const double *L, const double *Q,
+                                                         const uint32_t *meta,
+                                                         const unsigned int *bad, PosRec *X, R *P,
+                                                         R *Lo, R *Qo, int *slot)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N || bad[0] != ~0u || bad[1] != ~0u)
+        return;
+    const size_t o = i;
+    PosRec r;
+    r.x = x[3 * o];
+    r.y = x[3 * o + 1];
+    r.z = x[3 * o + 2];
+    r.id = (uint32_t)i;
+    r.meta = meta[i];
+    X[i] = r;
+    slot[i] = i;
+    for (int k = 0; k < 3; k++)
+        P[3 * o + k] = p ? (R)p[3 * o + k] : (R)0;
+    if (!Lo)
+        return;
+    for (int k = 0; k < 3; k++)
+        Lo[3 * o + k] = L ? (R)L[3 * o + k] : (R)0;
+    double m[9];
+    for (int k = 0; k < 9; k++)
+        m[k] = Q ? Q[9 * o + k] : (k % 4 == 0 ? 1.0 : 0.0);
+    if constexpr (sizeof(R) == 8) {
+        for (int k = 0; k < 9; k++)
+            Qo[9 * o + k] = m[k];
+    } else {
+        double q[4];
+        mat_to_quat<double>(m, q);
+        reinterpret_cast<float4 *>(Qo)[i] =
+            make_float4((float)q[0], (float)q[1], (float)q[2], (float)q[3]);
+    }
+}
+
+// the state of the current slots as FP64 arrays by original index (null
+// outputs are skipped; a null Q or L gives the bead integrator's identity and
+// zero).  Mixed: quaternions as matrices, normalised in FP64 first (the
+// stored FP32 norm is 1 only to FP32 rounding).  Rows of 24 and 72 B land at
+// random places, so the writes are partial lines; even so the kernel is a
+// small part of the copy that follows it (1,048,576 particles: 151 MB, 2.7 ms
+// at the link's rate).
+template <class R>
+__global__ void __launch_bounds__(256) k_state_by_id(int N, const PosRec *X, const R *p, const R *Q,
+                                                     const R *L, double *ox, double *op, double *oQ,
+                                                     double *oL)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= N)
+        return;
+    const PosRec r = X[s];
+    const size_t o = r.id;
+    if (ox) {
+        ox[3 * o] = r.x;
+        ox[3 * o + 1] = r.y;
+        ox[3 * o + 2] = r.z;
+    }
+    if (op)
+        for (int k = 0; k < 3; k++)
+            op[3 * o + k] = (double)p[3 * (size_t)s + k];
+    if (oL)
+        for (int k = 0; k < 3; k++)
+            oL[3 * o + k] = L ? (double)L[3 * (size_t)s + k] : 0.0;
+    if (!oQ)
+        return;
+    double m[9];
+    for (int k = 0; k < 9; k++)
+        m[k] = k % 4 == 0 ? 1.0 : 0.0;
+    if (Q) {
+        if constexpr (sizeof(R) == 8) {
+            for (int k = 0; k < 9; k++)
+                m[k] = Q[9 * (size_t)s + k];
+        } else {
+            const float4 q = reinterpret_cast<const float4 *>(Q)[s];
+            const double w = q.x, x = q.y, y = q.z, z = q.w;
+            const double inv = 1.0 / sqrt(w * w + x * x + y * y + z * z);
+            quat_to_mat<double>(w * inv, x * inv, y * inv, z * inv, m);
+        }
+    }
+    for (int k = 0; k < 9; k++)
+        oQ[9 * o + k] = m[k];
 }
 
 // a host array by original index (width values per particle, FP64) into the
@@ -3069,37 +3182,6 @@ __global__ void k_by_id_to_slots(const PosRec *X, int N, const double *in, R *ou
     const size_t o = X[s].id;
     for (int k = 0; k < width; k++)
         out[(size_t)width * s + k] = (R)in[width * o + k];
-}
-
-// host matrices (FP64, 9 per particle, slot order) into the mixed engine's
-// quaternions; Shepperd's method in FP64, rounded once
-__global__ void k_mats_to_quats(const double *in, int N, float *out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N)
-        return;
-    double m[9], q[4];
-    for (int k = 0; k < 9; k++)
-        m[k] = in[9 * (size_t)i + k];
-    mat_to_quat<double>(m, q);
-    reinterpret_cast<float4 *>(out)[i] = make_float4((float)q[0], (float)q[1], (float)q[2], (float)q[3]);
-}
-
-// the mixed engine's quaternions as FP64 rotation matrices (9 per particle,
-// slot order), normalised in FP64 first (the stored FP32 norm is 1 only to
-// FP32 rounding)
-__global__ void k_quats_to_mats(const float *in, int N, double *out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N)
-        return;
-    const float4 q = reinterpret_cast<const float4 *>(in)[i];
-    const double w = q.x, x = q.y, y = q.z, z = q.w;
-    const double inv = 1.0 / sqrt(w * w + x * x + y * y + z * z);
-    double m[9];
-    quat_to_mat<double>(w * inv, x * inv, y * inv, z * inv, m);
-    for (int k = 0; k < 9; k++)
-        out[9 * (size_t)i + k] = m[k];
 }
 
 // new (replica << 8 | type) words for the current slots from an array by
