@@ -56,6 +56,7 @@ struct BindArgs {
     uint32_t key0, key1;
     unsigned long long draw;
     int draw_epoch; // 1: the draw counter is the force-evaluation count (steps)
+    int ep_off;     // 1: that count already includes this evaluation (list steps)
     StepCtl *ctl;
     // 0: BindingModelSingle(on_rate, off_rate); 1: the species-table form of
     // BindingModelBinary / BindingModelTernary: species[patch] in 1..3,
@@ -73,13 +74,13 @@ struct BindArgs {
 __device__ __forceinline__ void bind_status(const BindArgs &b, unsigned bit)
 {
     atomicOr(&b.ctl->status, bit);
-    atomicMin(&b.ctl->fail_epoch, b.ctl->epoch);
+    atomicMin(&b.ctl->fail_epoch, b.ctl->epoch - b.ep_off);
 }
 
 // 53-bit uniform in [0, 1) of Philox4x32-10 at {root, draw lo, draw hi, k}
 __device__ __forceinline__ double bind_uniform(const BindArgs &b, int root, int k)
 {
-    const unsigned long long draw = b.draw_epoch ? b.ctl->epoch : b.draw;
+    const unsigned long long draw = b.draw_epoch ? b.ctl->epoch - b.ep_off : b.draw;
     const U4 o = philox4x32_10(
         U4{(uint32_t)root, (uint32_t)draw, (uint32_t)(draw >> 32), (uint32_t)k}, b.key0, b.key1);
     return ((double)(o.a >> 5) * 67108864.0 + (double)(o.b >> 6)) * (1.0 / 9007199254740992.0);

@@ -176,7 +176,8 @@ struct mdx_engine {
     bool list_eager = false; // an eager list step ran since the last list build
     GraphSlot graphs[2];     // per current state buffer
     Buf nbr, nbrc, nn, bcell; // neighbour list (column-major, per-block compact copy)
-    Buf dslot;           // drift maxima slots (NDSLOT), cleared by k_decide
+    Buf dslot;           // drift maxima slots, NDSLOT per state buffer
+    Buf head, link, utot, usync; // k_upkeep
     hipEvent_t prof_mid = nullptr;  // recorded between walk and finish while profiling
     hipEvent_t prof_mid2 = nullptr; // recorded between patch and integrate while profiling
     bool last_split = false;       // the last gather launch used the split form
@@ -483,6 +484,9 @@ static int build_grid(mdx_engine *e)
     if ((rc2 = dalloc(e, e->count, sizeof(int) * (size_t)(e->ncells + 1))))
         return rc2;
     HIPCHK(hipMemsetAsync(e->count.p, 0, sizeof(int) * (size_t)(e->ncells + 1), e->stream));
+    if ((rc2 = dalloc(e, e->head, sizeof(int) * (size_t)(e->ncells + 1))))
+        return rc2;
+    HIPCHK(hipMemsetAsync(e->head.p, 0, sizeof(int) * (size_t)(e->ncells + 1), e->stream));
     if ((rc2 = dalloc(e, e->start, sizeof(int) * (size_t)(e->ncells + 1))))
         return rc2;
     const int nb = (e->ncells + 1023) / 1024;
@@ -635,38 +639,41 @@ template <class R> static KArgs<R> make_args(mdx_engine *e)
     if (e->bind_on)
         a.rl2w = a.rl2; // every type pair can bind: one list radius (max_check + skin)
     a.skin = e->skin;
-    a.dslot = (unsigned int *)e->dslot.p;
+    // (a moving kernel fills the slots of the buffer it writes)
+    a.dslot = e->dslot.p ? (unsigned int *)e->dslot.p + NDSLOT * n : nullptr;
+    a.head = (int *)e->head.p;
+    a.link = (int *)e->link.p;
+    a.utot = (unsigned long long *)e->utot.p;
+    a.usync = (unsigned int *)e->usync.p;
     return a;
 }
 
 // scan + fill + per-cell ordering of the cell list built by the binning of
-// the current slots (cells: the binning's cell of each slot; gate: run only
-// when a list rebuild was requested)
-static int finish_bins(mdx_engine *e, const StepCtl *gate = nullptr, const int *cells = nullptr)
+// the current slots
+static int finish_bins(mdx_engine *e)
 {
     const int n = e->ncells;
     const int nb = (n + 1023) / 1024;
-    if (!cells)
-        cells = (const int *)e->cell[e->cur].p;
+    const int *cells = (const int *)e->cell[e->cur].p;
     hipLaunchKernelGGL(k_scan1, dim3(nb), dim3(256), 0, e->stream, (const int *)e->count.p,
-                       (int *)e->start.p, (int *)e->bsum.p, n, gate);
+                       (int *)e->start.p, (int *)e->bsum.p, n);
     hipLaunchKernelGGL(k_scan3, dim3(nb), dim3(256), 0, e->stream, (int *)e->count.p,
-                       (int *)e->start.p, (const int *)e->bsum.p, n, gate);
+                       (int *)e->start.p, (const int *)e->bsum.p, n);
     hipLaunchKernelGGL(k_fill, dim3(nblk(e->N)), dim3(256), 0, e->stream, e->N, cells,
-                       (const int *)e->rank.p, (const int *)e->start.p, (int *)e->list.p, gate);
+                       (const int *)e->rank.p, (const int *)e->start.p, (int *)e->list.p);
     hipLaunchKernelGGL(k_cellsort, dim3(nblk(e->N)), dim3(256), 0, e->stream, e->N, cells,
                        (const int *)e->rank.p, (const int *)e->start.p, (int *)e->list.p,
-                       (const PosRec *)e->X[e->cur].p, gate);
+                       (const PosRec *)e->X[e->cur].p);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
 
-// cell counts of the current slots into cells (gate as above)
-template <class R> static int count_current(mdx_engine *e, int *cells, const StepCtl *gate)
+// cell counts of the current slots
+template <class R> static int count_current(mdx_engine *e)
 {
     KArgs<R> a = make_args<R>(e);
-    a.celln = cells;
-    hipLaunchKernelGGL(k_bin<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, a, gate);
+    a.celln = (int *)e->cell[e->cur].p;
+    hipLaunchKernelGGL(k_bin<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -677,7 +684,7 @@ template <class R> static int bin_current(mdx_engine *e)
     int rc = build_grid(e);
     if (rc)
         return rc;
-    if (!e->counted && (rc = count_current<R>(e, (int *)e->cell[e->cur].p, nullptr)))
+    if (!e->counted && (rc = count_current<R>(e)))
         return rc;
     if ((rc = finish_bins(e)))
         return rc;
@@ -691,107 +698,117 @@ template <class R> static int bin_current(mdx_engine *e)
 template <class R, int MODE>
 static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode);
 
+// split form of a force evaluation: walk, patch kernel, integrator
 template <class R, int MODE>
-static int launch_gather(mdx_engine *e, const double *noise_dev, int lmode = 0)
+static int launch_split(mdx_engine *e, KArgs<R> &a, int lmode, bool bead_list)
 {
-    if (e->bind_on && (MODE == M_PRIME || MODE == M_STEP || MODE == M_FUSED))
-        return launch_bind_step<R, MODE>(e, noise_dev, lmode);
-    KArgs<R> a = make_args<R>(e);
-    a.noise = noise_dev;
-    a.lmode = lmode;
-    // split form: patch systems, and list steps of the bead integrator (walk,
-    // then the integrator kernel; no patch kernel)
-    const bool bead_list = MODE == M_BEAD && lmode && e->use_walkc;
-    const bool split = e->use_split && ((a.has_patches && (MODE == M_PRIME || MODE == M_STEP ||
-                                                           MODE == M_FUSED || MODE == M_CONS)) ||
-                                        bead_list);
-    if (split) {
-        int rc;
-        // list steps of the compacted walk hold every candidate of a position
-        // with at most kmax list entries (its candidates are among them)
-        const bool list_walk = lmode && e->use_walkc;
-        a.pcap = list_walk ? std::max(PMAXG, e->kmax) : PMAXG;
-        if ((rc = dalloc(e, e->Fw, 3 * e->rsz() * (size_t)e->N)) ||
-            (rc = dalloc(e, e->ncand, 4 * (size_t)e->N)) ||
-            (rc = dalloc(e, e->cand, 4 * (size_t)a.pcap * e->N)))
-            return rc;
-        if (e->use_compact && (rc = dalloc(e, e->Tp, 3 * e->rsz() * (size_t)e->N)))
-            return rc;
-        a.Fw = (R *)e->Fw.p;
-        a.ncand = (int *)e->ncand.p;
-        a.cand = (int *)e->cand.p;
-        a.Tp = (R *)e->Tp.p;
-        // positions per patch block: as many as keep about 512 blocks
-        int pblk = 256;
-        while (pblk < PBLK && (long long)e->N / (2 * pblk) >= 512)
-            pblk *= 2;
-        if (e->pblk > 0)
-            pblk = e->pblk;
-        // fused form (list steps): the walk integrates the particles without
-        // patch candidates, the patch kernel the others
-        const bool fuse_ok = e->use_fuse == 1 ||
-                             (e->use_fuse == 2 && (!a.has_patches || 4LL * e->n_patchy <= e->N));
-        const bool fuse = lmode && e->use_walkc && fuse_ok && e->use_compact &&
-                          (MODE == M_FUSED || MODE == M_STEP || MODE == M_BEAD);
+    // (list steps and the fused form exist for the moving modes only, and the
+    // bead integrator has no patch kernels)
+    constexpr bool moves = MODE == M_FUSED || MODE == M_STEP || MODE == M_BEAD;
+    constexpr bool patches = MODE != M_BEAD;
+    int rc;
+    // list steps of the compacted walk hold every candidate of a position
+    // with at most kmax list entries (its candidates are among them)
+    const bool list_walk = lmode && e->use_walkc;
+    a.pcap = list_walk ? std::max(PMAXG, e->kmax) : PMAXG;
+    if ((rc = dalloc(e, e->Fw, 3 * e->rsz() * (size_t)e->N)) ||
+        (rc = dalloc(e, e->ncand, 4 * (size_t)e->N)) ||
+        (rc = dalloc(e, e->cand, 4 * (size_t)a.pcap * e->N)))
+        return rc;
+    if (e->use_compact && (rc = dalloc(e, e->Tp, 3 * e->rsz() * (size_t)e->N)))
+        return rc;
+    a.Fw = (R *)e->Fw.p;
+    a.ncand = (int *)e->ncand.p;
+    a.cand = (int *)e->cand.p;
+    a.Tp = (R *)e->Tp.p;
+    // positions per patch block: as many as keep about 512 blocks
+    int pblk = 256;
+    while (pblk < PBLK && (long long)e->N / (2 * pblk) >= 512)
+        pblk *= 2;
+    if (e->pblk > 0)
+        pblk = e->pblk;
+    // fused form (list steps): the walk integrates the particles without
+    // patch candidates, the patch kernel the others
+    const bool fuse_ok =
+        e->use_fuse == 1 || (e->use_fuse == 2 && (!a.has_patches || 4LL * e->n_patchy <= e->N));
+    const bool fuse = list_walk && fuse_ok && e->use_compact;
+    const dim3 grid(nblk(e->N)), blk(256), pgrid(nblk(e->N, pblk));
+    e->last_split = true;
+    if constexpr (moves) {
         if (fuse) {
-            hipLaunchKernelGGL((k_walkc<R, MODE, true>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                               a);
+            hipLaunchKernelGGL((k_walkc<R, MODE, true>), grid, blk, 0, e->stream, a);
             if (e->prof_mid)
                 HIPCHK(hipEventRecord(e->prof_mid, e->stream));
-            e->last_split = true;
-            if (!bead_list) {
-                hipLaunchKernelGGL((k_patch<R, MODE, true>), dim3(nblk(e->N, pblk)), dim3(256), 0,
-                                   e->stream, a, pblk);
+            if constexpr (patches) {
+                if (!bead_list)
+                    hipLaunchKernelGGL((k_patch<R, MODE, true>), pgrid, blk, 0, e->stream, a, pblk);
             }
             if (e->prof_mid2)
                 HIPCHK(hipEventRecord(e->prof_mid2, e->stream));
             HIPCHK(hipGetLastError());
             return MDX_OK;
         }
-        if (lmode && e->use_walkc) {
+        if (list_walk) {
             // no overflow kernel after the compacted form's patch kernel: a
             // position with more candidates than kmax stops the run
             KArgs<R> w = a;
             w.ovf_fatal = e->use_compact ? 1 : 0;
-            hipLaunchKernelGGL((k_walkc<R, MODE, false>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                               w);
-        } else
-            hipLaunchKernelGGL((k_walk<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
-        if (e->prof_mid)
-            HIPCHK(hipEventRecord(e->prof_mid, e->stream));
-        e->last_split = true;
-        if (bead_list) {
-            if (e->prof_mid2)
-                HIPCHK(hipEventRecord(e->prof_mid2, e->stream));
-            hipLaunchKernelGGL((k_integrate<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                               a);
-        } else if (e->use_compact) {
-            hipLaunchKernelGGL((k_patch<R, MODE, false>), dim3(nblk(e->N, pblk)), dim3(256), 0,
-                               e->stream, a, pblk);
+            hipLaunchKernelGGL((k_walkc<R, MODE, false>), grid, blk, 0, e->stream, w);
+        }
+    }
+    if constexpr (patches) {
+        if (!list_walk)
+            hipLaunchKernelGGL((k_walk<R, MODE>), grid, blk, 0, e->stream, a);
+    }
+    if (e->prof_mid)
+        HIPCHK(hipEventRecord(e->prof_mid, e->stream));
+    if constexpr (patches) {
+        if (e->use_compact) {
+            hipLaunchKernelGGL((k_patch<R, MODE, false>), pgrid, blk, 0, e->stream, a, pblk);
             // (list steps hold every candidate: no overflow kernel)
             if (!list_walk)
-                hipLaunchKernelGGL((k_patch_ovf<R, MODE>), dim3(std::min(nblk(e->N), 512u)),
-                                   dim3(256), 0, e->stream, a);
-            if (e->prof_mid2)
-                HIPCHK(hipEventRecord(e->prof_mid2, e->stream));
-            hipLaunchKernelGGL((k_integrate<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                               a);
-        } else {
-            if (e->prof_mid2)
-                HIPCHK(hipEventRecord(e->prof_mid2, e->stream));
-            hipLaunchKernelGGL((k_finish<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                               a);
+                hipLaunchKernelGGL((k_patch_ovf<R, MODE>), dim3(std::min(nblk(e->N), 512u)), blk, 0,
+                                   e->stream, a);
         }
-        HIPCHK(hipGetLastError());
-        return MDX_OK;
+    }
+    if (e->prof_mid2)
+        HIPCHK(hipEventRecord(e->prof_mid2, e->stream));
+    if (bead_list || e->use_compact) {
+        hipLaunchKernelGGL((k_integrate<R, MODE>), grid, blk, 0, e->stream, a);
+    } else if constexpr (patches) {
+        hipLaunchKernelGGL((k_finish<R, MODE>), grid, blk, 0, e->stream, a);
+    }
+    HIPCHK(hipGetLastError());
+    return MDX_OK;
+}
+
+template <class R, int MODE>
+static int launch_gather(mdx_engine *e, const double *noise_dev, int lmode = 0)
+{
+    if constexpr (MODE == M_PRIME || MODE == M_STEP || MODE == M_FUSED) {
+        if (e->bind_on)
+            return launch_bind_step<R, MODE>(e, noise_dev, lmode);
+    }
+    KArgs<R> a = make_args<R>(e);
+    a.noise = noise_dev;
+    a.lmode = lmode;
+    a.ep_off = lmode ? 1 : 0; // (list steps: k_upkeep has counted the evaluation)
+    // split form: patch systems, and list steps of the bead integrator (walk,
+    // then the integrator kernel; no patch kernel)
+    const bool bead_list = MODE == M_BEAD && lmode && e->use_walkc;
+    const bool split = e->use_split && ((a.has_patches && (MODE == M_PRIME || MODE == M_STEP ||
+                                                           MODE == M_FUSED || MODE == M_CONS)) ||
+                                        bead_list);
+    if constexpr (MODE != M_ENERGY) {
+        if (split)
+            return launch_split<R, MODE>(e, a, lmode, bead_list);
     }
     e->last_split = false;
     // (k_tile: no list mode, nothing to close)
     if (e->use_tiles && !lmode)
         hipLaunchKernelGGL((k_tile<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
     else
-        hipLaunchKernelGGL((k_gather<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                           a);
+        hipLaunchKernelGGL((k_gather<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -863,6 +880,12 @@ static void launch_small(mdx_engine *e, void (*k)(StepCtl *))
     hipLaunchKernelGGL(k, dim3(1), dim3(1), 0, e->stream, (StepCtl *)e->ctl.p);
 }
 
+static void call_begin(mdx_engine *e)
+{
+    hipLaunchKernelGGL(k_call_begin, dim3(1), dim3(NDSLOT), 0, e->stream, (StepCtl *)e->ctl.p,
+                       (unsigned int *)e->dslot.p, e->cur, e->integ == MDX_INTEG_ROTOR ? 1 : 0);
+}
+
 template <class R> static int do_prime(mdx_engine *e, const double *noise0)
 {
     int rc = bin_current<R>(e);
@@ -871,7 +894,7 @@ template <class R> static int do_prime(mdx_engine *e, const double *noise0)
     const double *nd;
     if ((rc = noise_upload(e, noise0, (size_t)e->N * 6, &nd)))
         return rc;
-    launch_small(e, k_set_call_base);
+    call_begin(e);
     if ((rc = launch_gather<R, M_PRIME>(e, nd)))
         return rc;
     e->cur ^= 1;
@@ -893,18 +916,28 @@ static int nbr_alloc(mdx_engine *e)
     if ((rc = dalloc(e, e->nbr, 4 * (size_t)e->kmax * e->N)) ||
         (rc = dalloc(e, e->nbrc, 4 * (size_t)e->kmax * nblk(e->N) * 256)) ||
         (rc = dalloc(e, e->nn, 4 * (size_t)e->N)) || (rc = dalloc(e, e->bcell, 4 * (size_t)e->N)) ||
-        (rc = dalloc(e, e->dslot, 4 * (size_t)NDSLOT)))
+        (rc = dalloc(e, e->dslot, 4 * (size_t)(2 * NDSLOT))) ||
+        (rc = dalloc(e, e->link, 4 * (size_t)e->N)) ||
+        (rc = dalloc(e, e->utot, 8 * (size_t)UP_MAXTOT)) ||
+        (rc = dalloc(e, e->usync, 4 * (size_t)UP_SYNC)))
         return rc;
     return MDX_OK;
 }
 
-// after a kernel that moved the particles in list mode (its blocks wrote
-// drift slots); epoch_inc: also count the step's force evaluation;
-// step_end: the list step's kernels are done (clears fresh)
-static int decide(mdx_engine *e, int epoch_inc, int step_end)
+// the displacement decision and, when it is due, the cell list of the current
+// slots for a new neighbour list (k_nbuild follows)
+template <class R> static int upkeep(mdx_engine *e)
 {
-    hipLaunchKernelGGL(k_decide, dim3(1), dim3(NDSLOT), 0, e->stream, (StepCtl *)e->ctl.p,
-                       (unsigned int *)e->dslot.p, e->skin, epoch_inc, step_end);
+    KArgs<R> a = make_args<R>(e);
+    unsigned int *d = (unsigned int *)e->dslot.p;
+    const int c = e->cur, p0 = (e->N + UP_CHUNK - 1) / UP_CHUNK;
+    // cells per scan ticket: at most UP_MAXTOT tickets
+    const long long per = ((long long)e->ncells + UP_MAXTOT - 1) / UP_MAXTOT;
+    const int cc = (int)((per + UP_CHUNK - 1) / UP_CHUNK) * UP_CHUNK;
+    const int p1 = (e->ncells + cc - 1) / cc;
+    hipLaunchKernelGGL(k_upkeep<R>, dim3(std::min(std::max(p0, p1), 512)), dim3(UP_T), 0, e->stream,
+                       a, (const unsigned int *)d + NDSLOT * c, d + NDSLOT * (c ^ 1), c, e->ncells,
+                       p0, p1, cc);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -943,16 +976,13 @@ static inline void mark(mdx_engine *e, hipEvent_t *ev, int s, int k)
         (void)hipEventRecord(ev[NEV * s + k], e->stream);
 }
 
-// the kernels of one list step (gated list upkeep, walk / patch / integrate,
-// displacement decision); no host state changes, so it can be captured
+// the kernels of one list step (displacement decision and list upkeep, walk /
+// patch / integrate); no host state changes, so it can be captured
 template <class R, int MODE>
 static int launch_list_step(mdx_engine *e, const double *nd, hipEvent_t *ev, int s)
 {
     int rc;
-    const StepCtl *gate = (const StepCtl *)e->ctl.p;
-    if ((rc = count_current<R>(e, (int *)e->bcell.p, gate)))
-        return rc;
-    if ((rc = finish_bins(e, gate, (const int *)e->bcell.p)))
+    if ((rc = upkeep<R>(e)))
         return rc;
     if ((rc = build_list<R>(e, (const int *)e->bcell.p, 1)))
         return rc;
@@ -961,15 +991,7 @@ static int launch_list_step(mdx_engine *e, const double *nd, hipEvent_t *ev, int
     e->prof_mid2 = ev ? ev[NEV * s + 3] : nullptr;
     rc = launch_gather<R, MODE>(e, nd, 1);
     e->prof_mid = e->prof_mid2 = nullptr;
-    if (rc)
-        return rc;
-    if (MODE != M_STEP) {
-        if ((rc = decide(e, 1, 1)))
-            return rc;
-    } else {
-        launch_small(e, k_step_end);
-    }
-    return MDX_OK;
+    return rc;
 }
 
 // a list step from a graph captured per state buffer (the kernels' arguments
@@ -1027,7 +1049,7 @@ static int enqueue_one(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, b
     const bool lm = e->skin > 0;
     mark(e, ev, s, 0);
     if (!lm) {
-        if (!e->counted && (rc = count_current<R>(e, (int *)e->cell[e->cur].p, nullptr)))
+        if (!e->counted && (rc = count_current<R>(e)))
             return rc;
         if ((rc = finish_bins(e)))
             return rc;
@@ -1045,7 +1067,7 @@ static int enqueue_one(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, b
     } else if (!e->list_valid || e->since_resort >= e->resort_every) {
         if ((rc = nbr_alloc(e)))
             return rc;
-        if (!e->counted && (rc = count_current<R>(e, (int *)e->cell[e->cur].p, nullptr)))
+        if (!e->counted && (rc = count_current<R>(e)))
             return rc;
         if ((rc = finish_bins(e)))
             return rc;
@@ -1064,7 +1086,8 @@ static int enqueue_one(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, b
                 return rc;
             if ((rc = build_list<R>(e, (const int *)e->cell[e->cur].p, 0)))
                 return rc;
-            launch_small(e, k_list_reset);
+            hipLaunchKernelGGL(k_list_reset, dim3(1), dim3(NDSLOT), 0, e->stream,
+                               (StepCtl *)e->ctl.p, (unsigned int *)e->dslot.p);
             e->list_eager = false;
             // list steps keep the slots and do not rewrite the slot map
             HIPCHK(hipMemcpyAsync(e->slot[e->cur ^ 1].p, e->slot[e->cur].p, 4 * (size_t)e->N,
@@ -1109,7 +1132,7 @@ template <class R> static int enqueue_rotor(mdx_engine *e, int nsteps, const dou
     // the first kernel reads the replica table and bins into the cell grid
     if ((rc = build_grid(e)))
         return rc;
-    launch_small(e, k_set_call_base);
+    call_begin(e);
     {
         KArgs<R> a = make_args<R>(e);
         // with a live list the drift counts toward its displacement bound;
@@ -1119,8 +1142,6 @@ template <class R> static int enqueue_rotor(mdx_engine *e, int nsteps, const dou
             HIPCHK(hipEventRecord(kev[0], e->stream));
         hipLaunchKernelGGL(k_kick_drift<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
         HIPCHK(hipGetLastError());
-        if (a.lmode && (rc = decide(e, 0, 0)))
-            return rc;
         if (kev)
             HIPCHK(hipEventRecord(kev[1], e->stream));
         e->cur ^= 1;
@@ -1167,7 +1188,7 @@ template <class R> static int enqueue_bead(mdx_engine *e, int nsteps, const doub
     int rc;
     if ((rc = build_grid(e)))
         return rc;
-    launch_small(e, k_set_call_base);
+    call_begin(e);
     for (int s = 0; s < nsteps; s++)
         if ((rc = enqueue_one<R, M_BEAD>(e, nd, ev, s, s + 1 == nsteps)))
             return rc;
@@ -1356,7 +1377,8 @@ void mdx_destroy(mdx_engine *e)
                    &e->dslot,   &e->Tp,      &e->bpoff,  &e->bowner, &e->bisbound, &e->bboundto,
                    &e->badj_n,  &e->badj_p,  &e->badj_s, &e->bF,     &e->bT,      &e->bscr,
                    &e->bnscr,   &e->bspecies, &e->bdtab, &e->bttab,  &e->btr4,
-                   &e->plpairs, &e->plmask, &e->dmeta};
+                   &e->plpairs, &e->plmask, &e->dmeta,  &e->head,   &e->link,
+                   &e->utot,    &e->usync};
     for (Buf *b : bufs)
         dfree(*b);
     for (hipEvent_t ev : e->pin_ev)
@@ -2299,6 +2321,7 @@ template <class R> static BindArgs bind_args(mdx_engine *e, unsigned long long d
     b.key0 = (uint32_t)e->seed;
     b.key1 = (uint32_t)(e->seed >> 32) ^ 0xB1D0B1D0u;
     b.draw = draw;
+    b.draw_epoch = b.ep_off = 0;
     b.ctl = (StepCtl *)e->ctl.p;
     b.table = e->bind_table;
     b.species = (const int *)e->bspecies.p;
@@ -2319,6 +2342,7 @@ static int launch_bind(mdx_engine *e, const KArgs<R> &a, unsigned long long draw
 {
     BindArgs b = bind_args<R>(e, draw);
     b.draw_epoch = draw_epoch;
+    b.ep_off = a.ep_off;
     hipLaunchKernelGGL(k_bind_clear, dim3(nblk(e->nh)), dim3(256), 0, e->stream, b.adj_n, e->nh);
     if (!cand) {
         hipLaunchKernelGGL(k_bind_screen<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, a, b,
@@ -2366,6 +2390,7 @@ static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode)
     KArgs<R> a = make_args<R>(e);
     a.noise = noise_dev;
     a.lmode = lmode;
+    a.ep_off = lmode ? 1 : 0; // (list steps: k_upkeep has counted the evaluation)
     const bool list_walk = lmode && e->use_walkc;
     a.pcap = list_walk ? std::max(PMAXG, e->kmax) : PMAXG;
     int rc;
@@ -2393,10 +2418,12 @@ static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode)
             if (e->np[ta] > 0 && e->np[tc] > 0)
                 w.active_mask |= 1ull << (ta * MAXT + tc);
     w.ovf_fatal = 1;
-    if (list_walk)
-        hipLaunchKernelGGL((k_walkc<R, MODE, false>), dim3(nblk(e->N)), dim3(256), 0, e->stream,
-                           w);
-    else
+    if constexpr (MODE == M_FUSED || MODE == M_STEP) {
+        if (list_walk)
+            hipLaunchKernelGGL((k_walkc<R, MODE, false>), dim3(nblk(e->N)), dim3(256), 0,
+                               e->stream, w);
+    }
+    if (!list_walk)
         hipLaunchKernelGGL((k_walk<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream, w);
     if (e->prof_mid)
         HIPCHK(hipEventRecord(e->prof_mid, e->stream));
@@ -2776,7 +2803,7 @@ static int list_pairs_t(mdx_engine *e, int *ij, long long cap, long long *npairs
     int rc;
     if ((rc = build_grid(e)) || (rc = nbr_alloc(e)))
         return rc;
-    if (!e->counted && (rc = count_current<R>(e, (int *)e->cell[e->cur].p, nullptr)))
+    if (!e->counted && (rc = count_current<R>(e)))
         return rc;
     if ((rc = finish_bins(e)) || (rc = build_list<R>(e, (const int *)e->cell[e->cur].p, 0)))
         return rc;

@@ -42,9 +42,12 @@ struct StepCtl {
                                   // bit3 binding capacity
     unsigned int pad;
     // neighbour list: rebuild flag, displacement bound since the last build
-    unsigned int rebuild; // 1: the next step rebuilds the list before its walk
+    unsigned int rebuild; // 1: this step's k_upkeep asked for a new list
     unsigned int nbuilds; // list builds so far
-    double D;             // sum over steps of the max drift since the last build
+    // sum over steps of the max drift since the last build; k_upkeep reads the
+    // entry of its state buffer and writes the other (every block of it reads,
+    // one writes)
+    double D[2];
     // a walk queued more than pcap patch candidates for some position (the
     // overflow kernel's gate; cleared by the integrator kernel after it)
     unsigned int ovf;
@@ -52,8 +55,9 @@ struct StepCtl {
     // the status is clear.  From then on no moving kernel advances a particle.
     unsigned long long fail_epoch;
     // 1: a list build has written nbr since the compacted walk last laid its
-    // entries out per block (the next compacted walk does so); cleared by the
-    // kernel that closes the list step (k_decide, k_step_end)
+    // entries out per block (this step's compacted walk does so).  A build
+    // outside a list step leaves 2; each list step's k_upkeep turns 2 into 1
+    // and 1 into 0 before its own build
     unsigned int fresh;
 };
 
@@ -103,8 +107,18 @@ template <class R> struct KArgs {
     // pairs that cannot interact through patches
     double rl2, rl2w, skin;
     // drift maxima of the moving kernels' blocks (float bits, atomic max into
-    // slot block % NDSLOT); k_decide reduces and clears them
+    // slot block % NDSLOT), one set per state buffer: a moving kernel fills the
+    // set of the buffer it writes (dslot), k_upkeep reads that of the buffer
+    // that is current and clears the other
     unsigned int *dslot;
+    // list steps count their force evaluation before it (k_upkeep): 1 there
+    int ep_off;
+    // k_upkeep's working arrays: per cell the first particle of its chain plus
+    // one (0: empty; all 0 between builds) and per particle the next one,
+    // tagged chunk totals of the scan, ticket and phase counters
+    int *head, *link;
+    unsigned long long *utot;
+    unsigned int *usync;
     // WCA (HSPotential)
     int wca;
     double wca_eps, wca_s6, wca_s12, wca_pl, wca_pl2, wca_pl2lo;
@@ -281,7 +295,7 @@ template <class R> __device__ __forceinline__ void rotate(R dt, const R I[3], R 
 template <class R> __device__ __forceinline__ void raise_status(const KArgs<R> &a, unsigned bit)
 {
     atomicOr(&a.ctl->status, bit);
-    atomicMin(&a.ctl->fail_epoch, a.ctl->epoch);
+    atomicMin(&a.ctl->fail_epoch, a.ctl->epoch - a.ep_off);
 }
 
 // |f| of one term above the guard (the reference prints "force too big" and
@@ -306,7 +320,7 @@ template <class R> __device__ __forceinline__ bool stopped(const KArgs<R> &a)
 template <class R>
 __device__ __forceinline__ void load_noise(const KArgs<R> &a, uint32_t o, int ncomp, R out[6])
 {
-    unsigned long long ep = a.ctl->epoch;
+    const unsigned long long ep = a.ctl->epoch - a.ep_off;
     if (a.noise) {
         const double *row = a.noise + (size_t)(ep - a.ctl->call_base) * (size_t)a.N * ncomp +
                             (size_t)o * ncomp;
@@ -522,7 +536,7 @@ __device__ __forceinline__ void for_each_near(const KArgs<R> &a, const DevRep &r
 
 // block max of the drift into one of NDSLOT slots (atomic max on the float
 // bits, which order like the values for drifts >= 0; a non-finite drift
-// counts as infinite, so it forces a rebuild); k_decide reduces the slots
+// counts as infinite, so it forces a rebuild); k_upkeep reduces the slots
 constexpr int NDSLOT = 64;
 template <class R> __device__ __forceinline__ void drift_bound(const KArgs<R> &a, float d)
 {
@@ -1209,20 +1223,10 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
         bin_particle(a, s, rp, xn, a.celln);
 }
 
-// the first kernel after a list build clears the request and the bound
-template <class R> __device__ __forceinline__ void list_built(const KArgs<R> &a)
-{
-    if (a.lmode && blockIdx.x == 0 && threadIdx.x == 0 && a.ctl->rebuild) {
-        a.ctl->rebuild = 0u;
-        a.ctl->D = 0.0;
-    }
-}
-
 // one thread per cell-list position (list mode: per slot)
 template <class R, int MODE> __global__ void __launch_bounds__(256) k_gather(KArgs<R> a)
 {
     __shared__ int plist[PMAX * 256];
-    list_built(a);
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     float drift = 0.f;
     if (s < a.N)
@@ -1236,7 +1240,6 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_gather(KAr
 // split form: the neighbour walk ...
 template <class R, int MODE> __global__ void __launch_bounds__(256) k_walk(KArgs<R> a)
 {
-    list_built(a);
     const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (s >= a.N)
         return;
@@ -1270,7 +1273,6 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 4 && !INT) ? 6 : 1) k_walkc
     __shared__ R pf[256 * 3];
     __shared__ int pj[256];
     __shared__ int wsum[4];
-    list_built(a);
     const int tid = threadIdx.x;
     const int base = xcd_block(blockIdx.x, gridDim.x) * 256;
     const int s = base + tid;
@@ -1728,6 +1730,7 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_integrate(
 // memory instead.  NB_CAP: 800 (38 KB of LDS, 4 blocks per CU) for sparse
 // systems, 1152 (50 KB, 3 blocks) where an x-row of cells holds many
 // particles (the host picks it from the mean particles per row).
+constexpr int UP_SYNC = 4;     // k_upkeep: ticket counter, then done counts per phase
 constexpr int NB_W = 16;        // own x-rows of a block walked from LDS
 constexpr int NB_CAP_S = 800;   // staged particles per z offset (sparse)
 constexpr int NB_CAP_D = 1152;  // (dense)
@@ -1785,6 +1788,9 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
         atomicAdd(&a.ctl->nbuilds, 1u);
         a.ctl->fresh = 1u;
     }
+    // k_upkeep's counters and chains as it expects them next time
+    if (blockIdx.x == 0 && tid < UP_SYNC)
+        a.usync[tid] = 0u;
     const int p0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x;
     const int pos = p0 + tid;
     const int plast = min(p0 + (int)blockDim.x, a.N) - 1;
@@ -1796,6 +1802,7 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
         xi = a.X[s];
         c = cells[s];
         a.bcell[s] = c;
+        a.head[c] = 0;
         if (pos == p0) {
             ends[0] = (int)(xi.meta >> 8);
             ends[1] = c;
@@ -2290,10 +2297,8 @@ template <class R> __global__ void __launch_bounds__(256) k_kick_drift(KArgs<R> 
 }
 
 // binning of the current positions in place (after an upload or a reorder)
-template <class R> __global__ void __launch_bounds__(256) k_bin(KArgs<R> a, const StepCtl *gate)
+template <class R> __global__ void __launch_bounds__(256) k_bin(KArgs<R> a)
 {
-    if (gate && !gate->rebuild)
-        return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.N)
         return;
@@ -2360,20 +2365,13 @@ __device__ __forceinline__ void scan3_block(int *count, int *start, const int *b
         start[n] = off + bsum[b];
 }
 
-// gate: when non-null, each kernel runs only if a list rebuild was requested
-__global__ void __launch_bounds__(256) k_scan1(const int *count, int *start, int *bsum, int n,
-                                               const StepCtl *gate)
+__global__ void __launch_bounds__(256) k_scan1(const int *count, int *start, int *bsum, int n)
 {
-    if (gate && !gate->rebuild)
-        return;
     scan1_block(count, start, bsum, n, blockIdx.x);
 }
 
-__global__ void __launch_bounds__(256) k_scan3(int *count, int *start, const int *bsum, int n,
-                                               const StepCtl *gate)
+__global__ void __launch_bounds__(256) k_scan3(int *count, int *start, const int *bsum, int n)
 {
-    if (gate && !gate->rebuild)
-        return;
     scan3_block(count, start, bsum, n, blockIdx.x, gridDim.x);
 }
 
@@ -2384,10 +2382,8 @@ __device__ __forceinline__ void fill_one(const int *cell, const int *rank, const
 }
 
 __global__ void __launch_bounds__(256) k_fill(int N, const int *cell, const int *rank,
-                                              const int *start, int *list, const StepCtl *gate)
+                                              const int *start, int *list)
 {
-    if (gate && !gate->rebuild)
-        return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < N)
         fill_one(cell, rank, start, list, i);
@@ -2420,11 +2416,8 @@ __device__ __forceinline__ void cellsort_one(const int *cell, const int *rank, c
 }
 
 __global__ void __launch_bounds__(256) k_cellsort(int N, const int *cell, const int *rank,
-                                                  const int *start, int *list, const PosRec *X,
-                                                  const StepCtl *gate)
+                                                  const int *start, int *list, const PosRec *X)
 {
-    if (gate && !gate->rebuild)
-        return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < N)
         cellsort_one(cell, rank, start, list, X, i);
@@ -2436,56 +2429,252 @@ __global__ void k_epoch_inc(StepCtl *ctl)
         ctl->epoch += 1;
 }
 
-// the last kernel of a list step that moves nothing (M_STEP): the step's
-// force evaluation is counted, and the compacted walk has laid out any new list
-__global__ void k_step_end(StepCtl *ctl)
+// a list was just built outside a list step, at the current positions: no
+// rebuild pending, bound 0, no drift since (one wave)
+__global__ void __launch_bounds__(64) k_list_reset(StepCtl *ctl, unsigned int *dslot)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        ctl->epoch += 1;
-        ctl->fresh = 0u;
-    }
-}
-
-// a list was just built at the current positions: no rebuild pending, bound 0
-__global__ void k_list_reset(StepCtl *ctl)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        ctl->rebuild = 0u;
-        ctl->D = 0.0;
-    }
-}
-
-// the grid max of the block drifts of the kernel before is added to the
-// displacement bound D; a list rebuild is requested once 2 D reaches the skin
-// (a pair within reach now was within reach + skin at the build).
-// epoch_inc: also count the step's force evaluation; step_end: the list
-// step's kernels are done (the compacted walk has laid out any new list)
-__global__ void __launch_bounds__(64) k_decide(StepCtl *ctl, unsigned int *dslot, double skin,
-                                               int epoch_inc, int step_end)
-{
-    // one wave: each lane takes and clears one slot
-    float m = __uint_as_float(dslot[threadIdx.x]);
-    dslot[threadIdx.x] = 0u;
-    for (int o = 32; o > 0; o >>= 1)
-        m = fmaxf(m, __shfl_xor(m, o));
+    dslot[threadIdx.x] = dslot[NDSLOT + threadIdx.x] = 0u;
     if (threadIdx.x == 0) {
-        // margin for the rounding of the drift and of the FP64 position update
-        const double D = ctl->D + (double)m * (1 + 1e-6) + 1e-9;
-        ctl->D = D;
-        if (2 * D >= skin)
-            ctl->rebuild = 1u;
-        if (epoch_inc)
-            ctl->epoch += 1;
-        if (step_end)
-            ctl->fresh = 0u;
+        ctl->rebuild = 0u;
+        ctl->D[0] = ctl->D[1] = 0.0;
+        ctl->fresh = 2u;
     }
 }
 
-
-__global__ void k_set_call_base(StepCtl *ctl)
+// start of a call (one wave).  rotor: the state buffer changes twice between
+// the last k_upkeep of a call (its M_STEP kernel moves nothing) and the first
+// of the next, so the bound is handed to the entry that one reads, and the
+// drift slots, all counted by then, are cleared
+__global__ void __launch_bounds__(64) k_call_begin(StepCtl *ctl, unsigned int *dslot, int cur,
+                                                   int rotor)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0)
+    if (rotor && dslot)
+        dslot[threadIdx.x] = dslot[NDSLOT + threadIdx.x] = 0u;
+    if (threadIdx.x == 0) {
         ctl->call_base = ctl->epoch;
+        if (rotor)
+            ctl->D[cur ^ 1] = ctl->D[cur];
+    }
+}
+
+// ------------------------------------------------------------- list upkeep
+// One launch in place of seven (displacement decision, binning, two scan
+// kernels, fill, per-cell order, step count): an idle launch costs 2.5 to 4
+// us, and about nine list steps in ten rebuild nothing.
+//
+// Every block reduces the drift slots and takes the decision itself: the
+// maximum of the last moving kernel is added to the displacement bound D, and
+// a list rebuild is due once 2 D reaches the skin (a pair within reach now was
+// within reach + skin at the build).
+//
+// On a rebuild the blocks then work through tickets: binning (a chunk of
+// particles each), the scan of the cell counts (a chunk of cells each) and the
+// placing of the particles.  A ticket of one phase waits for all tickets of
+// the phase before.  Tickets are handed out in order, so whatever a block
+// waits for is held by a block that runs, however few blocks are resident:
+// every wait ends.  What one phase writes and another reads goes through
+// agent-scope loads and stores (through the XCDs' own L2s to memory), and a
+// block counts its ticket done after its stores have completed; no block
+// needs an L2 write-back, which made an earlier form of this with fences
+// eight times slower than separate kernels.
+//
+// Binning chains the particles of a cell (head, link) as well as counting
+// them; placing walks a particle's chain and counts the smaller original
+// indices, so the particles of a cell are listed in ascending original index
+// whatever the order of the atomics -- the order the gather's and the list's
+// floating-point sums depend on -- without a sorting pass.
+constexpr int UP_T = 1024;           // threads per block
+constexpr int UP_U = 4;              // particles (cells) per thread and round
+constexpr int UP_CHUNK = UP_T * UP_U; // particles per ticket
+constexpr int UP_MAXTOT = UP_T;      // most chunks of the scan
+
+template <class T> __device__ __forceinline__ T agent_load(const T *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T> __device__ __forceinline__ void agent_store(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// sum of v over the block (UP_T threads), and v's exclusive prefix
+__device__ __forceinline__ int block_scan(int v, int *sh, int &prefix)
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int s = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(s, o);
+        if (lane >= o)
+            s += t;
+    }
+    __syncthreads(); // (sh may still be read by the previous round)
+    if (lane == 63)
+        sh[wv] = s;
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < UP_T / 64; w++) {
+        before += w < wv ? sh[w] : 0;
+        all += sh[w];
+    }
+    prefix = before + s - v;
+    return all;
+}
+
+// dsl: the drift slots of the current state buffer, dslc: those to clear;
+// cur: that buffer; p0, p1: tickets of a particle phase and of the scan; cc:
+// cells per scan ticket (a multiple of UP_CHUNK)
+template <class R>
+__global__ void __launch_bounds__(UP_T) k_upkeep(KArgs<R> a, const unsigned int *dsl,
+                                                 unsigned int *dslc, int cur, int ncells, int p0,
+                                                 int p1, int cc)
+{
+    __shared__ int sh[UP_T / 64];
+    __shared__ int sdue, stick;
+    const int tid = threadIdx.x;
+    if (tid < 64) {
+        float m = __uint_as_float(dsl[tid]);
+        for (int o = 32; o > 0; o >>= 1)
+            m = fmaxf(m, __shfl_xor(m, o));
+        if (tid == 0) {
+            // margin for the rounding of the drift and of the FP64 position update
+            const double D = a.ctl->D[cur] + (double)m * (1 + 1e-6) + 1e-9;
+            const int due = 2 * D >= a.skin;
+            sdue = due;
+            if (blockIdx.x == 0) {
+                a.ctl->D[cur ^ 1] = due ? 0.0 : D;
+                a.ctl->rebuild = due;
+                a.ctl->fresh = a.ctl->fresh == 2u ? 1u : 0u;
+                a.ctl->epoch += 1;
+            }
+        }
+        if (blockIdx.x == 0)
+            dslc[tid] = 0u;
+    }
+    __syncthreads();
+    if (!sdue)
+        return;
+    const unsigned int tag = a.ctl->nbuilds + 1u;
+    const int tickets = 2 * p0 + p1;
+    for (;;) {
+        if (tid == 0)
+            stick = (int)atomicAdd(&a.usync[0], 1u);
+        __syncthreads();
+        const int t = stick;
+        if (t >= tickets)
+            return;
+        const int phase = t < p0 ? 0 : (t < p0 + p1 ? 1 : 2);
+        if (phase > 0) {
+            const unsigned int want = phase == 1 ? p0 : p1;
+            if (tid == 0)
+                while (agent_load(&a.usync[phase]) < want)
+                    __builtin_amdgcn_s_sleep(2);
+            __syncthreads();
+        }
+        if (phase == 0) {
+            const int lo = t * UP_CHUNK + tid;
+            int c[UP_U], old[UP_U];
+#pragma unroll
+            for (int u = 0; u < UP_U; u++) {
+                const int i = lo + u * UP_T;
+                c[u] = -1;
+                if (i < a.N) {
+                    const PosRec x = a.X[i];
+                    const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[x.meta >> 8];
+                    const int cx = axis_cell(x.x, rp.nc[0], rp.l[0]);
+                    const int cy = axis_cell(x.y, rp.nc[1], rp.l[1]);
+                    const int cz = axis_cell(x.z, rp.nc[2], rp.l[2]);
+                    c[u] = rp.coff + cx + rp.nc[0] * (cy + rp.nc[1] * cz);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < UP_U; u++)
+                if (c[u] >= 0) {
+                    old[u] = atomicExch(&a.head[c[u]], lo + u * UP_T + 1);
+                    atomicAdd(&a.count[c[u]], 1);
+                }
+#pragma unroll
+            for (int u = 0; u < UP_U; u++)
+                if (c[u] >= 0) {
+                    agent_store(&a.bcell[lo + u * UP_T], c[u]);
+                    agent_store(&a.link[lo + u * UP_T], old[u]);
+                }
+        } else if (phase == 1) {
+            const int k = t - p0, first = k * cc;
+            int *start = const_cast<int *>(a.start);
+            // the chunk's total, then the totals before it, then its starts
+            int sum = 0;
+            for (int b = first; b < min(first + cc, ncells); b += UP_CHUNK)
+#pragma unroll
+                for (int u = 0; u < UP_U; u++) {
+                    const int c = b + tid * UP_U + u;
+                    sum += c < ncells ? agent_load(&a.count[c]) : 0;
+                }
+            int run;
+            const int total = block_scan(sum, sh, run);
+            if (tid == 0)
+                agent_store(&a.utot[k], ((unsigned long long)tag << 32) | (unsigned int)total);
+            int before = 0;
+            if (tid < k) {
+                unsigned long long v;
+                while ((unsigned int)((v = agent_load(&a.utot[tid])) >> 32) != tag)
+                    __builtin_amdgcn_s_sleep(1);
+                before = (int)(unsigned int)v;
+            }
+            int base = block_scan(before, sh, run);
+            for (int b = first; b < min(first + cc, ncells); b += UP_CHUNK) {
+                int v[UP_U], s = 0;
+#pragma unroll
+                for (int u = 0; u < UP_U; u++) {
+                    const int c = b + tid * UP_U + u;
+                    v[u] = c < ncells ? agent_load(&a.count[c]) : 0;
+                    s += v[u];
+                }
+                const int all = block_scan(s, sh, run);
+                run += base;
+#pragma unroll
+                for (int u = 0; u < UP_U; u++) {
+                    const int c = b + tid * UP_U + u;
+                    if (c < ncells) {
+                        agent_store(&start[c], run);
+                        a.count[c] = 0;
+                    }
+                    run += v[u];
+                }
+                base += all;
+            }
+            if (k == p1 - 1 && tid == 0)
+                start[ncells] = base;
+        } else {
+            const int lo = (t - p0 - p1) * UP_CHUNK + tid;
+            int c[UP_U], j[UP_U], at[UP_U];
+#pragma unroll
+            for (int u = 0; u < UP_U; u++)
+                c[u] = lo + u * UP_T < a.N ? agent_load(&a.bcell[lo + u * UP_T]) : -1;
+#pragma unroll
+            for (int u = 0; u < UP_U; u++)
+                if (c[u] >= 0) {
+                    j[u] = agent_load(&a.head[c[u]]);
+                    at[u] = agent_load(&a.start[c[u]]);
+                }
+#pragma unroll
+            for (int u = 0; u < UP_U; u++)
+                if (c[u] >= 0) {
+                    const int i = lo + u * UP_T;
+                    const uint32_t id = a.X[i].id;
+                    for (int q = j[u]; q != 0;) {
+                        if (q - 1 != i)
+                            at[u] += a.X[q - 1].id < id ? 1 : 0;
+                        q = agent_load(&a.link[q - 1]);
+                    }
+                    const_cast<int *>(a.list)[at[u]] = i;
+                }
+        }
+        // the ticket's stores are complete before it counts as done
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0 && phase < 2)
+            atomicAdd(&a.usync[phase + 1], 1u);
+    }
 }
 
 // ---------------------------------------------------- parity entry points
