@@ -124,8 +124,8 @@ struct mdx_engine {
     // 0 the smaller, 1 the larger (MDX_NBDENSE)
     int nb_dense = -1;
     // walk / patch / integrator kernels (1) or one kernel per step (0); by
-    // default the one-kernel form up to SPLIT_MIN_N particles, where launches
-    // dominate the step (MDX_SPLIT=0/1 forces either)
+    // default the one-kernel form for small systems, where launches and chains
+    // of dependent work dominate the step (MDX_SPLIT=0/1 forces either)
     int use_split = 1;
     // neighbour list: skin > 0 enables it for mdx_step (MDX_SKIN), kmax slots per
     // particle (MDX_KMAX), state re-sorted into cell order every resort_every
@@ -554,6 +554,8 @@ template <class R> static KArgs<R> make_args(mdx_engine *e)
         a.np[t] = t < e->ntypes ? e->np[t] : 0;
         a.pstart[t] = t < e->ntypes ? e->pstart[t] : 0;
     }
+    for (int t = 0; t < e->ntypes; t++)
+        a.npat += e->np[t];
     for (int k = 0; k < MAXT * MAXT; k++)
         a.rstart[k] = k < (int)e->rstart.size() ? e->rstart[k] : 0;
     a.active_mask = e->active_mask;
@@ -804,6 +806,22 @@ static int launch_gather(mdx_engine *e, const double *noise_dev, int lmode = 0)
             return launch_split<R, MODE>(e, a, lmode, bead_list);
     }
     e->last_split = false;
+    if constexpr (MODE == M_FUSED || MODE == M_STEP || MODE == M_BEAD) {
+        if (lmode && e->use_walkc) {
+            // 16 positions per block while that leaves CUs idle (1,000
+            // tetrahedral particles, mixed: 32.7 us per step against 35.9 with
+            // 32), then 32 (8,000: 35.4 against 35.8; 16,000 in FP64: 37.5
+            // against 48.2)
+            if (e->N <= 4096)
+                hipLaunchKernelGGL((k_cstep<R, MODE, 16, 128>), dim3(nblk(e->N, 16)), dim3(128), 0,
+                                   e->stream, a);
+            else
+                hipLaunchKernelGGL((k_cstep<R, MODE, 32, 128>), dim3(nblk(e->N, 32)), dim3(128), 0,
+                                   e->stream, a);
+            HIPCHK(hipGetLastError());
+            return MDX_OK;
+        }
+    }
     // (k_tile: no list mode, nothing to close)
     if (e->use_tiles && !lmode)
         hipLaunchKernelGGL((k_tile<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
@@ -1286,10 +1304,12 @@ int mdx_create(const mdx_desc *d, mdx_engine **out)
     e->seed = d->seed;
     e->device = d->device;
     e->N = (int)N;
-    // measured on tetrahedral systems (FP64 / mixed): the one-kernel form is
-    // 5-14 % faster at 4,096-65,536 particles and 36 % slower at 262,144
-    constexpr long long SPLIT_MIN_N = 100000;
-    e->use_split = N > SPLIT_MIN_N;
+    // the one-kernel form while its blocks are all resident: FP64 us per step
+    // (tetrahedral / condensate) 54.7 / 44.8 against 58.7 / 44.7 split at
+    // 32,000 particles, 82 / 62 against 60 / 47 at 50,000; mixed 39 / 33
+    // against 56 / 42 at 32,000, 54.5 / 45.4 against 55.7 / 43.8 at 50,000
+    const long long split_min = e->prec == MDX_PREC_FP64 ? 32768 : 45000;
+    e->use_split = N > split_min;
     if (const char *t = std::getenv("MDX_TILES"))
         e->use_tiles = std::atoi(t) != 0;
     if (const char *t = std::getenv("MDX_PBLK"))

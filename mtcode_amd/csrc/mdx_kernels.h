@@ -126,6 +126,7 @@ template <class R> struct KArgs {
     int has_patches;
     int np[MAXT];
     int pstart[MAXT];
+    int npat; // patches of all types
     int rstart[MAXT * MAXT];
     unsigned long long active_mask; // bit ta * MAXT + tc: type pair with a nonzero row
     const double *pdirs;
@@ -562,6 +563,65 @@ template <class R> struct Acc {
     bool bad; // a term of this particle was above the force guard
 };
 
+// The type tables of the patch code in LDS, filled once per block.  Indexed per
+// lane from the kernel arguments or global memory they cost a dependent load
+// for each use inside loops of a few iterations, most of the walk's and the
+// patch kernel's time where few waves hide it (a list step of 4,096
+// particles: walk 18 us of latency, patch kernel 12 us).
+constexpr int MAXPT = MAXT * MAXP; // patches of all types
+struct ScreenTab {
+    float4 dir[MAXPT]; // body-frame directions, type-major
+    unsigned char np[MAXT], pstart[MAXT];
+};
+struct PatchTab : ScreenTab {
+    double dird[MAXPT * 3];
+    int rstart[MAXT * MAXT];
+};
+template <class R> __device__ __forceinline__ void load_tab(const KArgs<R> &a, ScreenTab &t)
+{
+    if (!a.pdirs_f)
+        return;
+    const int tid = threadIdx.x;
+    if (tid < MAXT) {
+        t.np[tid] = (unsigned char)a.np[tid];
+        t.pstart[tid] = (unsigned char)a.pstart[tid];
+    }
+    if (tid < a.npat)
+        t.dir[tid] = make_float4(a.pdirs_f[3 * tid], a.pdirs_f[3 * tid + 1], a.pdirs_f[3 * tid + 2], 0.f);
+}
+template <class R> __device__ __forceinline__ void load_tab(const KArgs<R> &a, PatchTab &t)
+{
+    if (!a.pdirs_f)
+        return;
+    load_tab(a, (ScreenTab &)t);
+    for (int k = threadIdx.x; k < 3 * a.npat; k += blockDim.x)
+        t.dird[k] = a.pdirs[k];
+    if (threadIdx.x < MAXT * MAXT)
+        t.rstart[threadIdx.x] = a.rstart[threadIdx.x];
+}
+
+// bit k: patch k of type ty, whose particle has the orientation q, passes the
+// FP32 cone screen sign * (n . u) > scr (u a unit vector)
+__device__ __forceinline__ uint32_t cone_mask(const ScreenTab &tb, int ty, const float q[9],
+                                              const float u[3], float sign, float scr)
+{
+    const float v[3] = {q[0] * u[0] + q[1] * u[1] + q[2] * u[2],
+                        q[3] * u[0] + q[4] * u[1] + q[5] * u[2],
+                        q[6] * u[0] + q[7] * u[1] + q[8] * u[2]};
+    const int np = tb.np[ty], p0 = tb.pstart[ty];
+    uint32_t m = 0;
+    // two at a time: their LDS reads overlap (a type without a second one
+    // reads its neighbour in the table)
+    for (int k = 0; k < np; k += 2) {
+        const float4 d0 = tb.dir[p0 + k], d1 = tb.dir[min(p0 + k + 1, MAXPT - 1)];
+        const float s0 = d0.x * v[0] + d0.y * v[1] + d0.z * v[2];
+        const float s1 = d1.x * v[0] + d1.y * v[1] + d1.z * v[2];
+        m |= (sign * s0 > scr ? 1u : 0u) << k;
+        m |= (k + 1 < np && sign * s1 > scr ? 2u : 0u) << k;
+    }
+    return m;
+}
+
 // roles of a patch pair: "a" = lower original index, exchanged when its type
 // is higher (GeneralPatch rows exist for ta <= tc; the potential is symmetric)
 __device__ __forceinline__ bool patch_roles(uint32_t oi, int ti, uint32_t oj, int tj, int &ta,
@@ -580,10 +640,14 @@ __device__ __forceinline__ bool patch_roles(uint32_t oi, int ti, uint32_t oj, in
 }
 
 // all patch pairs between particle i and neighbour slot j
-// (LangevinR.cpp:923-1044, potentialtheta.h:517-750)
+// (LangevinR.cpp:923-1044, potentialtheta.h:517-750).  The cone screens of
+// both sides come first, as bit masks, and only the passing patch pairs (one,
+// nearly always) are evaluated: lanes of a wave whose pairs bind through
+// different patches evaluate them together, not one patch pair after the
+// other as a loop over all of them does.
 template <class R, int MODE>
-__device__ __forceinline__ void patch_pair(const KArgs<R> &a, const DevRep &rp, const PosRec &xi,
-                                           int ti, const R *qi, int j, Acc<R> &acc)
+__device__ __forceinline__ void patch_pair(const KArgs<R> &a, const PatchTab &tb, const DevRep &rp,
+                                           const PosRec &xi, int ti, const R *qi, int j, Acc<R> &acc)
 {
     constexpr bool FP64 = sizeof(R) == 8;
     const PosRec xj = a.X[j];
@@ -600,31 +664,32 @@ __device__ __forceinline__ void patch_pair(const KArgs<R> &a, const DevRep &rp, 
     load_orient(a.Q, (size_t)j, qj);
     const R *qa = i_is_a ? qi : qj;
     const R *qc = i_is_a ? qj : qi;
-    // body-frame components of u screen the cone tests; the decisions are
-    // then taken on the reference's own FP64 expressions
-    const R ur[3] = {(R)u[0], (R)u[1], (R)u[2]};
-    const R va[3] = {qa[0] * ur[0] + qa[1] * ur[1] + qa[2] * ur[2],
-                     qa[3] * ur[0] + qa[4] * ur[1] + qa[5] * ur[2],
-                     qa[6] * ur[0] + qa[7] * ur[1] + qa[8] * ur[2]};
-    const R vc[3] = {qc[0] * ur[0] + qc[1] * ur[1] + qc[2] * ur[2],
-                     qc[3] * ur[0] + qc[4] * ur[1] + qc[5] * ur[2],
-                     qc[6] * ur[0] + qc[7] * ur[1] + qc[8] * ur[2]};
-    const int npa = a.np[ta], npc = a.np[tc];
-    const double *da = a.pdirs + 3 * a.pstart[ta];
-    const double *dc = a.pdirs + 3 * a.pstart[tc];
-    const int rowbase = rp.prow + a.rstart[ta * MAXT + tc];
-    const R scr = (R)a.costm_screen;
-    for (int ia = 0; ia < npa; ia++) {
-        const R s1 = -((R)da[3 * ia] * va[0] + (R)da[3 * ia + 1] * va[1] + (R)da[3 * ia + 2] * va[2]);
-        if (!(s1 > scr))
-            continue;
+    // the screens; the decisions are then taken on the reference's own FP64
+    // expressions
+    const float uf[3] = {(float)u[0], (float)u[1], (float)u[2]};
+    float qs[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+        qs[k] = (float)qa[k];
+    const float scr = (float)a.costm_screen_f;
+    const uint32_t ma = cone_mask(tb, ta, qs, uf, -1.f, scr);
+    if (!ma)
+        return;
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+        qs[k] = (float)qc[k];
+    const uint32_t mc = cone_mask(tb, tc, qs, uf, 1.f, scr);
+    const int npc = tb.np[tc];
+    const double *da = tb.dird + 3 * tb.pstart[ta];
+    const double *dc = tb.dird + 3 * tb.pstart[tc];
+    const int rowbase = rp.prow + tb.rstart[ta * MAXT + tc];
+    for (uint32_t m1 = mc ? ma : 0u; m1; m1 &= m1 - 1u) {
+        const int ia = __builtin_ctz(m1);
         double n1[3];
         lab_normal_exact(qa, da + 3 * ia, n1);
         const double a1 = -(n1[0] * u[0] + n1[1] * u[1] + n1[2] * u[2]);
-        for (int ib = 0; ib < npc; ib++) {
-            const R s2 = (R)dc[3 * ib] * vc[0] + (R)dc[3 * ib + 1] * vc[1] + (R)dc[3 * ib + 2] * vc[2];
-            if (!(s2 > scr))
-                continue;
+        for (uint32_t m2 = mc; m2; m2 &= m2 - 1u) {
+            const int ib = __builtin_ctz(m2);
             const PatchRow pr = a.prows[rowbase + ia * npc + ib];
             if (rij > pr.idist || !(a1 > pr.costm))
                 continue;
@@ -638,7 +703,6 @@ __device__ __forceinline__ void patch_pair(const KArgs<R> &a, const DevRep &rp, 
             if constexpr (FP64) {
                 e = kf2_pair_fp64(u, rij, n1, n2, a1, a2, pr, f, t1, t2);
             } else {
-                const float uf[3] = {(float)u[0], (float)u[1], (float)u[2]};
                 const float n1f[3] = {(float)n1[0], (float)n1[1], (float)n1[2]};
                 const float n2f[3] = {(float)n2[0], (float)n2[1], (float)n2[2]};
                 e = kf2_pair_fp32(uf, (float)rij, n1f, n2f, (float)a1, (float)a2,
@@ -742,30 +806,14 @@ __device__ __forceinline__ void wca_term(const KArgs<R> &a, const double d[3], d
 // walk uses it to hand over only candidates that can bind; every walk form
 // and the overflow path use this same screen, so they agree on the candidates.
 template <class R>
-__device__ __forceinline__ bool own_screen(const KArgs<R> &a, uint32_t oi, int ti, const float *qi,
-                                           const PosRec &xj, const double d[3], double r2s)
+__device__ __forceinline__ bool own_screen(const KArgs<R> &a, const ScreenTab &tb, int ti,
+                                           const float *qi, const double d[3], double r2s)
 {
-    const int tj = xj.meta & 255;
-    int ta, tc;
-    const bool i_is_a = patch_roles(oi, ti, xj.id, tj, ta, tc);
-    // u = (d / r), sign folded into the test below
+    // u = +d/r for role a, whose test is -(n . u); u = -d/r for role c, whose
+    // test is n . u: both are -(n . d/r)
     const float ri = rsqrtf((float)r2s);
     const float ur[3] = {(float)d[0] * ri, (float)d[1] * ri, (float)d[2] * ri};
-    const float v[3] = {qi[0] * ur[0] + qi[1] * ur[1] + qi[2] * ur[2],
-                        qi[3] * ur[0] + qi[4] * ur[1] + qi[5] * ur[2],
-                        qi[6] * ur[0] + qi[7] * ur[1] + qi[8] * ur[2]};
-    const int t = i_is_a ? ta : tc;
-    const int np = a.np[t];
-    const float *dd = a.pdirs_f + 3 * a.pstart[t];
-    const float scr = (float)a.costm_screen_f;
-    bool pass = false;
-    for (int k = 0; k < np; k++) {
-        const float sd = dd[3 * k] * v[0] + dd[3 * k + 1] * v[1] + dd[3 * k + 2] * v[2];
-        // u = +d/r for role a, whose test is -(n . u); u = -d/r for role c,
-        // whose test is n . u: both are -(n . d/r)
-        pass |= -sd > scr;
-    }
-    return pass;
+    return cone_mask(tb, ti, qi, ur, -1.f, (float)a.costm_screen_f) != 0u;
 }
 
 // the moved position of slot s into the next buffer (the whole record: a
@@ -791,11 +839,12 @@ __device__ __forceinline__ void store_position(const KArgs<R> &a, int s, const P
 // only (WCA force and patch candidates to global memory); PH_FINISH: the
 // patches from those candidates, topology and the integrator.  The split
 // keeps the register-heavy patch code out of the neighbour walk.
-// PH_INTEGRATE_F: as PH_INTEGRATE with the force given in fin and no patch
-// torque (a particle without patch candidates, integrated by the walk)
+// PH_INTEGRATE_F: as PH_INTEGRATE with the force and patch torque given in
+// fin (3 + 3); bad: one of the particle's terms was above the force guard
 template <class R, int MODE, int PH, class Trav>
-__device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *plist, Trav &&trav,
-                                                 float &drift, const R *fin = nullptr)
+__device__ __forceinline__ void process_particle(const KArgs<R> &a, const PatchTab *tb, int s,
+                                                 int *plist, Trav &&trav, float &drift,
+                                                 const R *fin = nullptr, bool bad = false)
 {
     constexpr bool FP64 = sizeof(R) == 8;
     const int i = a.lmode ? s : a.list[s];
@@ -843,7 +892,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
     // the candidates the split form hands over: those that pass the screen
     auto is_listed_candidate = [&](const PosRec &xj, int js, const double d[3], double r2s) -> bool {
         (void)js;
-        return is_patch_candidate(xj, r2s) && own_screen(a, oi, ti, qs, xj, d, r2s);
+        return is_patch_candidate(xj, r2s) && own_screen(a, *tb, ti, qs, d, r2s);
     };
     if (PH == PH_FINISH) {
         for (int k = 0; k < 3; k++)
@@ -851,7 +900,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
         const int npc = a.ncand[s];
         const int nq = npc < a.pcap ? npc : a.pcap;
         for (int q = 0; q < nq; q++)
-            patch_pair<R, MODE>(a, rp, xi, ti, qi, a.cand[(size_t)q * a.N + s], acc);
+            patch_pair<R, MODE>(a, *tb, rp, xi, ti, qi, a.cand[(size_t)q * a.N + s], acc);
         if (npc > a.pcap) {
             int seen = 0;
             trav(i, rp, [&](const PosRec &xj, int j) {
@@ -863,7 +912,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
                     !(MDX_WALK_SCREEN ? is_listed_candidate(xj, js, d, r2s) : is_patch_candidate(xj, r2s)))
                     return;
                 if (seen++ >= a.pcap)
-                    patch_pair<R, MODE>(a, rp, xi, ti, qi, js, acc);
+                    patch_pair<R, MODE>(a, *tb, rp, xi, ti, qi, js, acc);
             });
         }
     }
@@ -886,8 +935,9 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
     if (PH == PH_INTEGRATE_F) {
         for (int k = 0; k < 3; k++) {
             acc.F[k] = fin[k];
-            acc.T[k] = (R)0;
+            acc.T[k] = fin[3 + k];
         }
+        acc.bad = bad;
     }
     if (PH != PH_FINISH && !INTG && (a.wca || npi > 0)) {
         int npc = 0;
@@ -922,7 +972,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
         // -------- patches (LangevinR.cpp:911-1047), in neighbour-loop order
         const int nq = npc < PMAX ? npc : PMAX;
         for (int q = 0; q < nq; q++)
-            patch_pair<R, MODE>(a, rp, xi, ti, qi, plist[q * 256 + threadIdx.x], acc);
+            patch_pair<R, MODE>(a, *tb, rp, xi, ti, qi, plist[q * 256 + threadIdx.x], acc);
         if (npc > PMAX) {
             // dense neighbourhoods: a second traversal takes the rest in order
             int seen = 0;
@@ -933,7 +983,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
                 if (!(r2s < a.rmax2) || !is_patch_candidate(xj, r2s))
                     return;
                 if (seen++ >= PMAX)
-                    patch_pair<R, MODE>(a, rp, xi, ti, qi, j >= 0 ? j : a.slot[xj.id], acc);
+                    patch_pair<R, MODE>(a, *tb, rp, xi, ti, qi, j >= 0 ? j : a.slot[xj.id], acc);
             });
         }
     }
@@ -1227,11 +1277,14 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, int s, int *
 template <class R, int MODE> __global__ void __launch_bounds__(256) k_gather(KArgs<R> a)
 {
     __shared__ int plist[PMAX * 256];
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
+    __syncthreads();
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     float drift = 0.f;
     if (s < a.N)
         process_particle<R, MODE, PH_ALL>(
-            a, s, plist, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
+            a, &tb, s, plist, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
             drift);
     if ((MODE == M_FUSED || MODE == M_BEAD) && a.lmode)
         drift_bound(a, drift);
@@ -1240,12 +1293,15 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_gather(KAr
 // split form: the neighbour walk ...
 template <class R, int MODE> __global__ void __launch_bounds__(256) k_walk(KArgs<R> a)
 {
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
+    __syncthreads();
     const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (s >= a.N)
         return;
     float drift = 0.f;
     process_particle<R, MODE, PH_WALK>(
-        a, s, nullptr, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
+        a, &tb, s, nullptr, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
         drift);
 }
 
@@ -1273,6 +1329,8 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 4 && !INT) ? 6 : 1) k_walkc
     __shared__ R pf[256 * 3];
     __shared__ int pj[256];
     __shared__ int wsum[4];
+    __shared__ ScreenTab tb;
+    load_tab(a, tb);
     const int tid = threadIdx.x;
     const int base = xcd_block(blockIdx.x, gridDim.x) * 256;
     const int s = base + tid;
@@ -1333,16 +1391,16 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 4 && !INT) ? 6 : 1) k_walkc
             return false;
         wca_term<R, MODE>(a, d, r2s, xj.id, e0, e1, acc);
         const int to = xo.meta & 255;
-        if (!(a.has_patches && a.np[to] > 0 && r2s < a.maxd2))
+        if (!(a.has_patches && r2s < a.maxd2))
             return false;
         const int tj = xj.meta & 255;
-        if (a.np[tj] == 0)
+        if (tb.np[to] == 0 || tb.np[tj] == 0)
             return false;
         int ta, tc;
         patch_roles(xo.id, to, xj.id, tj, ta, tc);
         if (!((a.active_mask >> (ta * MAXT + tc)) & 1ull))
             return false;
-        return !MDX_WALK_SCREEN || own_screen(a, xo.id, to, qo, xj, d, r2s);
+        return own_screen(a, tb, to, qo, d, r2s);
     };
 
     R F[3] = {0, 0, 0};
@@ -1460,9 +1518,9 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 4 && !INT) ? 6 : 1) k_walkc
         }
         __syncthreads();
         if (tid < nint) {
-            const R fin[3] = {pf[3 * tid], pf[3 * tid + 1], pf[3 * tid + 2]};
+            const R fin[6] = {pf[3 * tid], pf[3 * tid + 1], pf[3 * tid + 2], 0, 0, 0};
             process_particle<R, MODE, PH_INTEGRATE_F>(
-                a, pj[tid], nullptr,
+                a, nullptr, pj[tid], nullptr,
                 [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); }, drift,
                 fin);
         }
@@ -1471,14 +1529,251 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 4 && !INT) ? 6 : 1) k_walkc
     }
 }
 
+// The whole list step of NPOS positions in one kernel of T threads, for small
+// systems (the engine has the sizes): there the launches and the longest chain
+// of dependent work bound the step, not the chip's width.
+// The block lays its list entries out back to back and evaluates WCA and the
+// own-patch screen, one entry per lane; each position sums its entries in list
+// order; its patch candidates are again laid out one per lane and added in
+// list order; then the positions are integrated by the block's first wave.
+// The sums are the one-lane kernel's (k_gather) in the same order, so the
+// results are the same bits while at most one patch pair of a particle pair
+// passes its cone tests.
+// A round of entries is a chain of dependent loads and LDS reads, 3.2 us with
+// as many lanes as positions and 6 rounds of them (tetrahedral fluid, 5.4
+// entries per position); with four to eight lanes per position 2.  Per block
+// of 64 positions and 256 lanes: 2.8 us to load the positions, 0.8 offsets,
+// 5.2 entries, 2.9 patch candidates, 2.2 integrator; k_gather's lanes, which
+// took their patch candidates in turn, 42 us for 4,096 particles.
+constexpr int CS_CAND = 8; // patch candidates per position and pass (more: more passes)
+template <class R, int MODE, int NPOS, int T>
+__global__ void __launch_bounds__(T) k_cstep(KArgs<R> a)
+{
+    static_assert(NPOS <= 64 && T >= 64 && T <= 256, "the first wave holds the positions");
+    __shared__ int off[NPOS];
+    __shared__ PosRec sx[NPOS];
+    __shared__ float sq[NPOS * 9]; // orientations in FP32 for the own-patch screen
+    __shared__ int sexc[NPOS * 2];
+    __shared__ unsigned char spl[NPOS], sbad[NPOS];
+    __shared__ unsigned char own[CS_CAND * NPOS > T ? CS_CAND * NPOS : T]; // owner of an entry
+    __shared__ R ent[T * 6]; // force (and torque) per lane
+    __shared__ int pj[T];
+    __shared__ int plist[CS_CAND * NPOS];
+    __shared__ int stotal;
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
+    const int tid = threadIdx.x;
+    const int base = xcd_block(blockIdx.x, gridDim.x) * NPOS;
+    const int s = base + tid;
+    const bool live = tid < NPOS && s < a.N;
+    const int n = live ? list_count(a, s) : 0;
+    const bool fb = n > a.kmax;
+    const int cnt = fb ? 0 : n;
+    PosRec xi;
+    if (live) {
+        xi = a.X[s];
+        sx[tid] = xi;
+        sbad[tid] = 0;
+        const bool ne = needs_exclusions(a, s);
+        sexc[2 * tid] = ne ? a.exc_off[xi.id] : 0;
+        sexc[2 * tid + 1] = ne ? a.exc_off[xi.id + 1] : 0;
+        spl[tid] = face_clear(a, rep_rec(a, xi.meta), xi);
+        if (MODE != M_BEAD && a.has_patches) {
+            R qm[9];
+            load_orient(a.Q, (size_t)s, qm);
+#pragma unroll
+            for (int k = 0; k < 9; k++)
+                sq[9 * tid + k] = (float)qm[k];
+        }
+    }
+    // exclusive scan of v over the positions (first wave); the total in stotal
+    auto scan = [&](int v) -> int {
+        int t = v;
+        if (tid < 64) {
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(t, o);
+                if (tid >= o)
+                    t += u;
+            }
+            if (tid == 63)
+                stotal = t;
+        }
+        return t - v;
+    };
+    // WCA of a pair into acc; true for a patch candidate that passes the
+    // own-patch screen
+    auto visit = [&](const PosRec &xo, const float *qo, int e0, int e1, bool pl,
+                     const PosRec &xj, Acc<R> &acc) -> bool {
+        const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xo.meta >> 8];
+        double d[3];
+        if (pl) {
+            d[0] = xo.x - xj.x;
+            d[1] = xo.y - xj.y;
+            d[2] = xo.z - xj.z;
+        } else {
+            min_image(a, rp, xo.x, xo.y, xo.z, xj, d);
+        }
+        const double r2s = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        if (!(r2s < a.rmax2))
+            return false;
+        wca_term<R, MODE>(a, d, r2s, xj.id, e0, e1, acc);
+        if constexpr (MODE == M_BEAD) {
+            return false;
+        } else {
+            if (!(a.has_patches && r2s < a.maxd2))
+                return false;
+            const int to = xo.meta & 255, tj = xj.meta & 255;
+            if (tb.np[to] == 0 || tb.np[tj] == 0)
+                return false;
+            int ta, tc;
+            patch_roles(xo.id, to, xj.id, tj, ta, tc);
+            return ((a.active_mask >> (ta * MAXT + tc)) & 1ull) && own_screen(a, tb, to, qo, d, r2s);
+        }
+    };
+
+    const int off0 = scan(cnt);
+    if (tid < NPOS)
+        off[tid] = off0;
+    __syncthreads();
+    const int total = stotal;
+    R F[3] = {0, 0, 0}, Tq[3] = {0, 0, 0};
+    bool bad = false;
+    int c0 = 0, more = 0; // patch candidates of a position taken by earlier passes
+    do {
+        int npc = 0;
+        auto take = [&](int j) {
+            if (npc >= c0 && npc < c0 + CS_CAND)
+                plist[(npc - c0) * NPOS + tid] = j;
+            npc++;
+        };
+        for (int r0 = 0; r0 < total; r0 += T) {
+            const int lo = max(off0, r0), hi = min(off0 + cnt, r0 + T);
+            for (int e2 = lo; e2 < hi; e2++)
+                own[e2 - r0] = (unsigned char)tid;
+            __syncthreads();
+            const int e = r0 + tid;
+            if (e < total) {
+                const int o = own[tid];
+                const int j = a.nbr[(size_t)(e - off[o]) * a.N + base + o];
+                const PosRec xj = a.X[j];
+                const PosRec xo = sx[o];
+                Acc<R> pa;
+                pa.F[0] = pa.F[1] = pa.F[2] = 0;
+                pa.bad = false;
+                const bool c = visit(xo, sq + 9 * o, sexc[2 * o], sexc[2 * o + 1], spl[o], xj, pa);
+                for (int k = 0; k < 3; k++)
+                    ent[3 * tid + k] = pa.F[k];
+                if (pa.bad)
+                    sbad[o] = 1;
+                pj[tid] = c ? j : -1;
+            }
+            __syncthreads();
+            // in list order, four reads at a time
+            for (int e2 = lo; e2 < hi; e2 += 4) {
+                R f[4][3];
+                int jc[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int q = min(e2 + u, hi - 1) - r0;
+                    for (int k = 0; k < 3; k++)
+                        f[u][k] = ent[3 * q + k];
+                    jc[u] = e2 + u < hi ? pj[q] : -1;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (c0 == 0 && e2 + u < hi)
+                        for (int k = 0; k < 3; k++)
+                            F[k] += f[u][k];
+                    if (jc[u] >= 0)
+                        take(jc[u]);
+                }
+            }
+        }
+        if (fb && live) {
+            // more entries than the list holds: the build's cells, in this lane
+            Acc<R> pa;
+            pa.F[0] = pa.F[1] = pa.F[2] = 0;
+            pa.bad = false;
+            const DevRep rp = rep_rec(a, xi.meta);
+            for_each_in_cells(a, rp, a.bcell[s], s, [&](const PosRec &xj, int j) {
+                if (visit(xi, sq + 9 * tid, sexc[2 * tid], sexc[2 * tid + 1], spl[tid], xj, pa))
+                    take(j);
+            });
+            if (c0 == 0)
+                for (int k = 0; k < 3; k++)
+                    F[k] = pa.F[k];
+            bad |= pa.bad;
+        }
+        if constexpr (MODE != M_BEAD) {
+            // this pass's patch candidates, one per lane
+            const int nq = max(0, min(npc - c0, CS_CAND));
+            __syncthreads(); // (own, ent and stotal have been read)
+            const int first = scan(nq);
+            if (tid < NPOS)
+                off[tid] = first;
+            for (int k = 0; k < nq; k++)
+                own[first + k] = (unsigned char)tid;
+            __syncthreads();
+            const int ncand = stotal;
+            for (int r0 = 0; r0 < ncand; r0 += T) {
+                const int e = r0 + tid;
+                if (e < ncand) {
+                    const int o = own[e];
+                    const PosRec xo = sx[o];
+                    const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xo.meta >> 8];
+                    R qo[9];
+                    load_orient(a.Q, (size_t)(base + o), qo);
+                    Acc<R> ea;
+                    for (int k = 0; k < 3; k++)
+                        ea.F[k] = ea.T[k] = 0;
+                    ea.bad = false;
+                    patch_pair<R, MODE>(a, tb, rp, xo, xo.meta & 255, qo,
+                                        plist[(e - off[o]) * NPOS + o], ea);
+                    for (int k = 0; k < 3; k++) {
+                        ent[6 * tid + k] = ea.F[k];
+                        ent[6 * tid + 3 + k] = ea.T[k];
+                    }
+                }
+                __syncthreads();
+                for (int e2 = max(first, r0); e2 < min(first + nq, r0 + T); e2++)
+                    for (int k = 0; k < 3; k++) {
+                        F[k] += ent[6 * (e2 - r0) + k];
+                        Tq[k] += ent[6 * (e2 - r0) + 3 + k];
+                    }
+                __syncthreads();
+            }
+            c0 += CS_CAND;
+            more = __syncthreads_or(npc > c0);
+            if (more) {
+                if (tid < NPOS)
+                    off[tid] = off0;
+                __syncthreads();
+            }
+        }
+    } while (more);
+    float drift = 0.f;
+    if (live) {
+        const R fin[6] = {F[0], F[1], F[2], Tq[0], Tq[1], Tq[2]};
+        process_particle<R, MODE, PH_INTEGRATE_F>(
+            a, nullptr, s, nullptr,
+            [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); }, drift, fin,
+            bad || sbad[tid]);
+    }
+    if (MODE == M_FUSED || MODE == M_BEAD)
+        drift_bound(a, drift);
+}
+
 // ... then the patch pairs, topology and the integrator
 template <class R, int MODE> __global__ void __launch_bounds__(256) k_finish(KArgs<R> a)
 {
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
+    __syncthreads();
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     float drift = 0.f;
     if (s < a.N)
         process_particle<R, MODE, PH_FINISH>(
-            a, s, nullptr, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
+            a, &tb, s, nullptr, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
             drift);
     if ((MODE == M_FUSED || MODE == M_BEAD) && a.lmode)
         drift_bound(a, drift);
@@ -1488,7 +1783,7 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_finish(KAr
 // the neighbours are walked again in walk order and the terms after the
 // first pcap candidates added to Fw / Tp (k_patch has added the others)
 template <class R, int MODE>
-__device__ __forceinline__ void patch_overflow(const KArgs<R> &a, int so)
+__device__ __forceinline__ void patch_overflow(const KArgs<R> &a, const PatchTab &tb, int so)
 {
     const int i = a.lmode ? so : a.list[so];
     const PosRec xi = a.X[i];
@@ -1520,11 +1815,11 @@ __device__ __forceinline__ void patch_overflow(const KArgs<R> &a, int so)
         patch_roles(xi.id, ti, xj.id, tj, ta, tc);
         if (!((a.active_mask >> (ta * MAXT + tc)) & 1ull))
             return;
-        if (MDX_WALK_SCREEN && !own_screen(a, xi.id, ti, qs, xj, d, r2s))
+        if (MDX_WALK_SCREEN && !own_screen(a, tb, ti, qs, d, r2s))
             return;
         const int js = j >= 0 ? j : a.slot[xj.id];
         if (seen++ >= a.pcap)
-            patch_pair<R, MODE>(a, rp, xi, ti, qi, js, acc);
+            patch_pair<R, MODE>(a, tb, rp, xi, ti, qi, js, acc);
     });
     for (int k2 = 0; k2 < 3; k2++) {
         a.Fw[3 * (size_t)so + k2] = acc.F[k2];
@@ -1552,6 +1847,8 @@ __global__ void __launch_bounds__(256) k_patch(KArgs<R> a, int pblk)
     __shared__ int off[PBLK + 1];
     __shared__ R ent[256 * 6];
     __shared__ int wsum[4];
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
     const int tid = threadIdx.x;
     const int base = xcd_block(blockIdx.x, gridDim.x) * pblk;
     // exclusive scan of min(ncand, pcap) in position order (position
@@ -1606,7 +1903,7 @@ __global__ void __launch_bounds__(256) k_patch(KArgs<R> a, int pblk)
             for (int k = 0; k < 3; k++)
                 ea.F[k] = ea.T[k] = 0;
             ea.bad = false;
-            patch_pair<R, MODE>(a, rp, xo, xo.meta & 255, qo, a.cand[(size_t)q * a.N + so], ea);
+            patch_pair<R, MODE>(a, tb, rp, xo, xo.meta & 255, qo, a.cand[(size_t)q * a.N + so], ea);
             for (int k = 0; k < 3; k++) {
                 ent[6 * tid + k] = ea.F[k];
                 ent[6 * tid + 3 + k] = ea.T[k];
@@ -1643,7 +1940,7 @@ __global__ void __launch_bounds__(256) k_patch(KArgs<R> a, int pblk)
         for (int k = 0; k < PER; k++) {
             const int so = base + k * 256 + tid;
             if (so < a.N && a.ncand[so] > a.pcap)
-                patch_overflow<R, MODE>(a, so);
+                patch_overflow<R, MODE>(a, tb, so);
         }
     if (INT) {
         // the positions with candidates, compacted into off[], integrated one
@@ -1672,7 +1969,7 @@ __global__ void __launch_bounds__(256) k_patch(KArgs<R> a, int pblk)
         for (int t = tid; t < cnt; t += 256) {
             float d = 0.f;
             process_particle<R, MODE, PH_INTEGRATE>(
-                a, off[t], nullptr,
+                a, nullptr, off[t], nullptr,
                 [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); }, d);
             drift = fmaxf(drift, d);
         }
@@ -1688,9 +1985,12 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_patch_ovf(
 {
     if (!a.ctl->ovf)
         return;
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
+    __syncthreads();
     for (int so = blockIdx.x * blockDim.x + threadIdx.x; so < a.N; so += gridDim.x * blockDim.x)
         if (a.ncand[so] > a.pcap)
-            patch_overflow<R, MODE>(a, so);
+            patch_overflow<R, MODE>(a, tb, so);
 }
 
 // ... and the topology terms and the integrator
@@ -1702,7 +2002,7 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_integrate(
     float drift = 0.f;
     if (s < a.N)
         process_particle<R, MODE, PH_INTEGRATE>(
-            a, s, nullptr, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
+            a, nullptr, s, nullptr, [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); },
             drift);
     if ((MODE == M_FUSED || MODE == M_BEAD) && a.lmode)
         drift_bound(a, drift);
@@ -2094,6 +2394,8 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_tile(KArgs
     __shared__ int hbase[TILE_HROWS + 1];
     __shared__ int hcell[TILE_HROWS];
     __shared__ int tinfo[8]; // use_lds, ya, nr, z, rep, nh
+    __shared__ PatchTab tb;
+    load_tab(a, tb); // (a barrier follows before its first use)
     const int s0 = blockIdx.x * blockDim.x;
     const int s1 = min(a.N, s0 + (int)blockDim.x);
     if (threadIdx.x == 0) {
@@ -2174,7 +2476,7 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_tile(KArgs
             return;
         const int ya = tinfo[1], nr = tinfo[2];
         float drift_unused = 0.f;
-        process_particle<R, MODE, PH_ALL>(a, s, plist, [&](int i, const DevRep &rq, auto &&fn) {
+        process_particle<R, MODE, PH_ALL>(a, &tb, s, plist, [&](int i, const DevRep &rq, auto &&fn) {
             const uint32_t self = a.X[i].id;
             const int c = a.cell[i] - rq.coff;
             const int cx = c % n0;
@@ -2214,7 +2516,7 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_tile(KArgs
     if (s >= s1)
         return;
     float drift_unused = 0.f;
-    process_particle<R, MODE, PH_ALL>(a, s, plist, [&](int i, const DevRep &rp, auto &&fn) {
+    process_particle<R, MODE, PH_ALL>(a, &tb, s, plist, [&](int i, const DevRep &rp, auto &&fn) {
         for_each_neighbor(a, rp, i, fn);
     }, drift_unused);
 }
