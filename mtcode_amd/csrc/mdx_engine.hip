@@ -79,6 +79,13 @@ struct Span {
     size_t bytes;
 };
 
+// list steps replayed as one graph while as many are left before the next
+// re-sort or the end of the call.  Even: the state buffers alternate, so the
+// graph ends on the buffer it began with.  Consecutive graphs are about 8 us
+// apart on the device, the kernels of one graph are not (4,096 particles: 33
+// us per step in graphs of one step)
+constexpr int GRAPH_STEPS = 8;
+
 struct GraphSlot {
     hipGraphExec_t exec = nullptr;
     std::vector<char> sig; // launch arguments it was captured with
@@ -174,7 +181,7 @@ struct mdx_engine {
     int use_fuse = 2;
     int n_patchy = 0; // particles whose type carries patches
     bool list_eager = false; // an eager list step ran since the last list build
-    GraphSlot graphs[2];     // per current state buffer
+    GraphSlot graphs[2][2];  // one step, GRAPH_STEPS steps; per current state buffer
     Buf nbr, nbrc, nn, bcell; // neighbour list (column-major, per-block compact copy)
     Buf dslot;           // drift maxima slots, NDSLOT per state buffer
     Buf head, link, utot, usync; // k_upkeep
@@ -1012,10 +1019,11 @@ static int launch_list_step(mdx_engine *e, const double *nd, hipEvent_t *ev, int
     return rc;
 }
 
-// a list step from a graph captured per state buffer (the kernels' arguments
-// differ only in which buffer is current); recaptured when the arguments
-// change.  The graph holds kernel nodes only (no memset or copy nodes).
-template <class R, int MODE> static int list_step_graph(mdx_engine *e)
+// steps list steps from a graph captured per state buffer (the kernels'
+// arguments differ only in which buffer is current); recaptured when the
+// arguments change.  The graph holds kernel nodes only (no memset or copy
+// nodes).
+template <class R, int MODE> static int list_step_graph(mdx_engine *e, int steps)
 {
     KArgs<R> a = make_args<R>(e);
     a.lmode = 1;
@@ -1028,15 +1036,21 @@ template <class R, int MODE> static int list_step_graph(mdx_engine *e)
     memcpy(sig.data(), &a, sizeof a);
     memcpy(sig.data() + sizeof a, form, sizeof form);
     memcpy(sig.data() + sizeof a + sizeof form, rates, sizeof rates);
-    GraphSlot &g = e->graphs[e->cur];
+    GraphSlot &g = e->graphs[steps > 1][e->cur];
     if (!g.exec || g.sig != sig) {
         if (g.exec) {
             HIPCHK(hipGraphExecDestroy(g.exec));
             g.exec = nullptr;
         }
         hipGraph_t graph = nullptr;
+        const int cur = e->cur;
         HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeRelaxed));
-        int rc = launch_list_step<R, MODE>(e, nullptr, nullptr, 0);
+        int rc = MDX_OK;
+        for (int k = 0; k < steps && !rc; k++) {
+            rc = launch_list_step<R, MODE>(e, nullptr, nullptr, 0);
+            e->cur ^= 1;
+        }
+        e->cur = cur;
         hipError_t ce = hipStreamEndCapture(e->stream, &graph);
         if (rc)
             return rc;
@@ -1060,10 +1074,13 @@ template <class R, int MODE> static int list_step_graph(mdx_engine *e)
 // With the list, a re-sort step does the same and then builds the list at
 // the new positions; the steps in between walk the list in place, and a
 // rebuild runs (gated kernels) whenever the displacement bound asks for it.
+// left: steps of this mode still to come in the call, this one included;
+// *done: how many were enqueued
 template <class R, int MODE>
-static int enqueue_one(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, bool last)
+static int enqueue_some(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, int left, int *done)
 {
     int rc;
+    *done = 1;
     const bool lm = e->skin > 0;
     mark(e, ev, s, 0);
     if (!lm) {
@@ -1121,15 +1138,18 @@ static int enqueue_one(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, b
         // replayed from a captured graph once an eager list step has run
         // with the same launch arguments (engine noise, not profiling)
         const bool graph = e->use_graph && !ev && !nd && MODE != M_STEP && e->list_eager;
-        if (graph)
-            rc = list_step_graph<R, MODE>(e);
-        else
+        if (graph) {
+            if (std::min(left, e->resort_every - e->since_resort) >= GRAPH_STEPS)
+                *done = GRAPH_STEPS;
+            rc = list_step_graph<R, MODE>(e, *done);
+        } else {
             rc = launch_list_step<R, MODE>(e, nd, ev, s);
+        }
         if (rc)
             return rc;
         e->list_eager = true;
-        e->cur ^= 1;
-        e->since_resort++;
+        e->cur ^= *done & 1;
+        e->since_resort += *done;
         e->binned = false;
         e->counted = false;
     }
@@ -1138,7 +1158,6 @@ static int enqueue_one(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, b
         mark(e, ev, s, 3);
     }
     mark(e, ev, s, 4);
-    (void)last;
     return MDX_OK;
 }
 
@@ -1165,10 +1184,9 @@ template <class R> static int enqueue_rotor(mdx_engine *e, int nsteps, const dou
         e->cur ^= 1;
         e->counted = !a.lmode;
     }
-    for (int s = 0; s < nsteps; s++) {
-        const bool last = s + 1 == nsteps;
-        rc = last ? enqueue_one<R, M_STEP>(e, nd, ev, s, last)
-                  : enqueue_one<R, M_FUSED>(e, nd, ev, s, last);
+    for (int s = 0, n; s < nsteps; s += n) {
+        rc = s + 1 == nsteps ? enqueue_some<R, M_STEP>(e, nd, ev, s, 1, &n)
+                             : enqueue_some<R, M_FUSED>(e, nd, ev, s, nsteps - 1 - s, &n);
         if (rc)
             return rc;
     }
@@ -1207,8 +1225,8 @@ template <class R> static int enqueue_bead(mdx_engine *e, int nsteps, const doub
     if ((rc = build_grid(e)))
         return rc;
     call_begin(e);
-    for (int s = 0; s < nsteps; s++)
-        if ((rc = enqueue_one<R, M_BEAD>(e, nd, ev, s, s + 1 == nsteps)))
+    for (int s = 0, n; s < nsteps; s += n)
+        if ((rc = enqueue_some<R, M_BEAD>(e, nd, ev, s, nsteps - s, &n)))
             return rc;
     e->steps_taken += nsteps;
     return MDX_OK;
@@ -1405,9 +1423,10 @@ void mdx_destroy(mdx_engine *e)
         if (ev)
             (void)hipEventDestroy(ev);
     pin_release(e);
-    for (GraphSlot &g : e->graphs)
-        if (g.exec)
-            (void)hipGraphExecDestroy(g.exec);
+    for (auto &per_count : e->graphs)
+        for (GraphSlot &g : per_count)
+            if (g.exec)
+                (void)hipGraphExecDestroy(g.exec);
     for (int b = 0; b < 2; b++) {
         dfree(e->X[b]);
         dfree(e->Q[b]);
