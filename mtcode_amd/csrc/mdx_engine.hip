@@ -186,7 +186,7 @@ struct mdx_engine {
     Buf dslot;           // drift maxima slots, NDSLOT per state buffer
     Buf head, link, utot, usync; // k_upkeep
     Buf arank, acount, absum;    // the analysis grids' cell lists
-    Buf alab;                    // cluster labels
+    Buf asorted, aedge, alab;    // positions in cell order, bin edges, cluster labels
     hipEvent_t prof_mid = nullptr;  // recorded between walk and finish while profiling
     hipEvent_t prof_mid2 = nullptr; // recorded between patch and integrate while profiling
     bool last_split = false;       // the last gather launch used the split form
@@ -1419,7 +1419,7 @@ void mdx_destroy(mdx_engine *e)
                    &e->bnscr,   &e->bspecies, &e->bdtab, &e->bttab,  &e->btr4,
                    &e->plpairs, &e->plmask, &e->dmeta,  &e->head,   &e->link,
                    &e->utot,    &e->usync,  &e->arank,  &e->acount, &e->absum,
-                   &e->alab};
+                   &e->asorted, &e->aedge,  &e->alab};
     for (Buf *b : bufs)
         dfree(*b);
     for (hipEvent_t ev : e->pin_ev)
@@ -1936,9 +1936,10 @@ int mdx_cell_assign(mdx_engine *e, int replica, const int n[3], int *cell_of)
 }
 
 // positions of replica r in original order (tmpx), their cells on an
-// n[0] x n[1] x n[2] grid (tmpi) and that grid's cell list (tmpi3: starts,
-// tmpi2: members in original order); a parity / analysis path, not the step
-static int custom_cells(mdx_engine *e, int replica, const int n[3])
+// n[0] x n[1] x n[2] grid (tmpi), that grid's cell list (tmpi3: starts, tmpi2:
+// members, in original order if ordered) and the positions in the list's order
+// (asorted, written before the ordering); a parity / analysis path, not the step
+static int custom_cells(mdx_engine *e, int replica, const int n[3], bool ordered)
 {
     const long long nc = (long long)n[0] * n[1] * n[2];
     if (nc > (1ll << 28))
@@ -1953,7 +1954,8 @@ static int custom_cells(mdx_engine *e, int replica, const int n[3])
     // lists of two grids took 0.8 ms for 100,003 particles)
     const int ncell = (int)nc, nb = (ncell + 1023) / 1024;
     if ((rc = dalloc(e, e->arank, 4 * (size_t)cnt)) || (rc = dalloc(e, e->acount, 4 * (size_t)ncell)) ||
-        (rc = dalloc(e, e->absum, 4 * (size_t)nb)))
+        (rc = dalloc(e, e->absum, 4 * (size_t)nb)) ||
+        (rc = dalloc(e, e->asorted, sizeof(PosRec) * (size_t)cnt)))
         return rc;
     HIPCHK(hipMemsetAsync(e->acount.p, 0, 4 * (size_t)ncell, e->stream));
     int *cell = (int *)e->tmpi.p, *start = (int *)e->tmpi3.p, *list = (int *)e->tmpi2.p;
@@ -1964,10 +1966,13 @@ static int custom_cells(mdx_engine *e, int replica, const int n[3])
                        (int *)e->absum.p, ncell);
     hipLaunchKernelGGL(k_scan3, dim3(nb), dim3(256), 0, e->stream, (int *)e->acount.p, start,
                        (const int *)e->absum.p, ncell);
-    hipLaunchKernelGGL(k_fill, dim3(nblk(cnt)), dim3(256), 0, e->stream, cnt, (const int *)cell,
-                       (const int *)e->arank.p, (const int *)start, list);
-    hipLaunchKernelGGL(k_cellsort, dim3(nblk(cnt)), dim3(256), 0, e->stream, cnt, (const int *)cell,
-                       (const int *)e->arank.p, (const int *)start, list, (const PosRec *)nullptr);
+    hipLaunchKernelGGL(k_fill_custom, dim3(nblk(cnt)), dim3(256), 0, e->stream,
+                       (const double *)e->tmpx.p, cnt, (const int *)cell, (const int *)e->arank.p,
+                       (const int *)start, list, (PosRec *)e->asorted.p);
+    if (ordered)
+        hipLaunchKernelGGL(k_cellsort, dim3(nblk(cnt)), dim3(256), 0, e->stream, cnt,
+                           (const int *)cell, (const int *)e->arank.p, (const int *)start, list,
+                           (const PosRec *)nullptr);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -1993,14 +1998,28 @@ int mdx_pair_histogram(mdx_engine *e, int replica, double max, double dx, long l
             return set_err(MDX_ERR_ARG, "max larger than the box");
     }
     int rc;
-    if ((rc = custom_cells(e, replica, n)) || (rc = dalloc(e, e->tmpll, 8 * (size_t)std::max(gs, 1))))
+    // edge[b]: the smallest squared distance in bin b or a later one, with the
+    // reference's floor(sqrt(d2) / dx)
+    auto bin_of = [&](double d2) { return std::floor(std::sqrt(d2) / dx); };
+    std::vector<double> edge((size_t)gs + 1, 0.0);
+    for (int k = 1; k <= gs; k++) {
+        double d2 = (k * dx) * (k * dx);
+        while (bin_of(d2) >= k)
+            d2 = std::nextafter(d2, 0.0);
+        while (bin_of(d2) < k)
+            d2 = std::nextafter(d2, HUGE_VAL);
+        edge[(size_t)k] = d2;
+    }
+    if ((rc = custom_cells(e, replica, n, false)) ||
+        (rc = dalloc(e, e->tmpll, 8 * (size_t)std::max(gs, 1))) ||
+        (rc = upload(e, e->aedge, edge.data(), edge.size())))
         return rc;
     HIPCHK(hipMemsetAsync(e->tmpll.p, 0, 8 * (size_t)std::max(gs, 1), e->stream));
     const int cnt = e->nper[replica];
-    hipLaunchKernelGGL(k_gcount, dim3(nblk(cnt)), dim3(256), 0, e->stream,
-                       (const double *)e->tmpx.p, cnt, b[0], b[1], b[2], e->periodic, n[0], n[1],
-                       n[2], (const int *)e->tmpi.p, (const int *)e->tmpi3.p,
-                       (const int *)e->tmpi2.p, dx, gs, (unsigned long long *)e->tmpll.p);
+    hipLaunchKernelGGL(k_gcount, dim3(nblk(cnt), 3), dim3(256), 8 * (size_t)(gs + 1) + 4 * (size_t)gs,
+                       e->stream, (const PosRec *)e->asorted.p, cnt, b[0], b[1], b[2], e->periodic,
+                       n[0], n[1], n[2], (const int *)e->tmpi3.p, (const double *)e->aedge.p,
+                       (float)(1.0 / dx), gs, (unsigned long long *)e->tmpll.p);
     HIPCHK(hipGetLastError());
     *nbins = gs;
     std::vector<long long> h((size_t)std::max(gs, 1));
@@ -2046,7 +2065,7 @@ static int pair_list(mdx_engine *e, int replica, const int n[3], double cut, Buf
     const int cnt = e->nper[replica];
     const double *b = &e->box[3 * replica];
     int rc;
-    if ((rc = custom_cells(e, replica, n)) || (rc = dalloc(e, e->tmpll, 8 * (size_t)(cnt + 1))) ||
+    if ((rc = custom_cells(e, replica, n, true)) || (rc = dalloc(e, e->tmpll, 8 * (size_t)(cnt + 1))) ||
         (rc = dalloc(e, e->partial, 4 * (size_t)cnt)))
         return rc;
     const double *X = (const double *)e->tmpx.p;
@@ -2119,14 +2138,13 @@ int mdx_clusters(mdx_engine *e, int replica, const int n[3], double cut, int ex_
     const int cnt = e->nper[replica];
     const double *b = &e->box[3 * replica];
     int rc;
-    if ((rc = custom_cells(e, replica, n)) || (rc = dalloc(e, e->alab, 4 * (size_t)cnt)))
+    if ((rc = custom_cells(e, replica, n, false)) || (rc = dalloc(e, e->alab, 4 * (size_t)cnt)))
         return rc;
     int *lab = (int *)e->alab.p;
     hipLaunchKernelGGL(k_cc_init, dim3(nblk(cnt)), dim3(256), 0, e->stream, lab, cnt);
-    hipLaunchKernelGGL(k_cc_pairs, dim3(nblk(cnt)), dim3(256), 0, e->stream,
-                       (const double *)e->tmpx.p, cnt, b[0], b[1], b[2], e->periodic, n[0], n[1],
-                       n[2], cut, (const int *)e->tmpi.p, (const int *)e->tmpi3.p,
-                       (const int *)e->tmpi2.p, ex_lo, ex_hi, lab);
+    hipLaunchKernelGGL(k_cc_pairs, dim3(nblk(cnt), 3), dim3(256), 0, e->stream,
+                       (const PosRec *)e->asorted.p, cnt, b[0], b[1], b[2], e->periodic, n[0], n[1],
+                       n[2], cut, (const int *)e->tmpi3.p, ex_lo, ex_hi, lab);
     hipLaunchKernelGGL(k_cc_flatten, dim3(nblk(cnt)), dim3(256), 0, e->stream, lab, cnt);
     HIPCHK(hipGetLastError());
     if ((rc = download(e, e->alab, labels, (size_t)cnt)))
