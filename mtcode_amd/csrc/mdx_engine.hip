@@ -184,7 +184,7 @@ struct mdx_engine {
     GraphSlot graphs[2][2];  // one step, GRAPH_STEPS steps; per current state buffer
     Buf nbr, nbrc, nn, bcell; // neighbour list (column-major, per-block compact copy)
     Buf dslot;           // drift maxima slots, NDSLOT per state buffer
-    Buf head, link, utot, usync; // k_upkeep
+    Buf bucket, head, link, utot, usync; // k_upkeep
     Buf arank, acount, absum;    // the analysis grids' cell lists
     Buf asorted, aedge, alab;    // positions in cell order, bin edges, cluster labels
     hipEvent_t prof_mid = nullptr;  // recorded between walk and finish while profiling
@@ -490,13 +490,17 @@ static int build_grid(mdx_engine *e)
     int rc2;
     if ((rc2 = upload(e, e->dreps, e->reps.data(), e->reps.size())))
         return rc2;
-    if ((rc2 = dalloc(e, e->count, sizeof(int) * (size_t)(e->ncells + 1))))
+    // (counts and starts in whole tiles of k_upkeep's scan)
+    const size_t padded = ((size_t)e->ncells + 1 + UP_SCAN - 1) / UP_SCAN * UP_SCAN;
+    if ((rc2 = dalloc(e, e->count, sizeof(int) * padded)))
         return rc2;
-    HIPCHK(hipMemsetAsync(e->count.p, 0, sizeof(int) * (size_t)(e->ncells + 1), e->stream));
+    HIPCHK(hipMemsetAsync(e->count.p, 0, sizeof(int) * padded, e->stream));
+    if ((rc2 = dalloc(e, e->bucket, sizeof(int) * UP_BUCKET * (size_t)(e->ncells + 1))))
+        return rc2;
     if ((rc2 = dalloc(e, e->head, sizeof(int) * (size_t)(e->ncells + 1))))
         return rc2;
     HIPCHK(hipMemsetAsync(e->head.p, 0, sizeof(int) * (size_t)(e->ncells + 1), e->stream));
-    if ((rc2 = dalloc(e, e->start, sizeof(int) * (size_t)(e->ncells + 1))))
+    if ((rc2 = dalloc(e, e->start, sizeof(int) * padded)))
         return rc2;
     const int nb = (e->ncells + 1023) / 1024;
     if (nb > 1024 * 1024)
@@ -652,6 +656,7 @@ template <class R> static KArgs<R> make_args(mdx_engine *e)
     a.skin = e->skin;
     // (a moving kernel fills the slots of the buffer it writes)
     a.dslot = e->dslot.p ? (unsigned int *)e->dslot.p + NDSLOT * n : nullptr;
+    a.bucket = (unsigned int *)e->bucket.p;
     a.head = (int *)e->head.p;
     a.link = (int *)e->link.p;
     a.utot = (unsigned long long *)e->utot.p;
@@ -957,14 +962,22 @@ template <class R> static int upkeep(mdx_engine *e)
 {
     KArgs<R> a = make_args<R>(e);
     unsigned int *d = (unsigned int *)e->dslot.p;
-    const int c = e->cur, p0 = (e->N + UP_CHUNK - 1) / UP_CHUNK;
-    // cells per scan ticket: at most UP_MAXTOT tickets
-    const long long per = ((long long)e->ncells + UP_MAXTOT - 1) / UP_MAXTOT;
-    const int cc = (int)((per + UP_CHUNK - 1) / UP_CHUNK) * UP_CHUNK;
-    const int p1 = (e->ncells + cc - 1) / cc;
-    hipLaunchKernelGGL(k_upkeep<R>, dim3(std::min(std::max(p0, p1), 512)), dim3(UP_T), 0, e->stream,
-                       a, (const unsigned int *)d + NDSLOT * c, d + NDSLOT * (c ^ 1), c, e->ncells,
-                       p0, p1, cc);
+    // particles per ticket: one per thread while that makes at most 512 tickets
+    const int U = e->N <= 512 * UP_T ? 1 : 2;
+    const int c = e->cur, p0 = (e->N + U * UP_T - 1) / (U * UP_T);
+    // cells per scan ticket: at most UP_MAXTOT tickets.  The cells include the
+    // one past the end, whose start is the particle count
+    const int n = e->ncells + 1;
+    const int per = (n + UP_MAXTOT - 1) / UP_MAXTOT;
+    const int cc = (per + UP_SCAN - 1) / UP_SCAN * UP_SCAN;
+    const int p1 = (n + cc - 1) / cc;
+    const dim3 grid(std::min(std::max(p0, p1), 512)), blk(UP_T);
+    const unsigned int *now = d + NDSLOT * c;
+    unsigned int *next = d + NDSLOT * (c ^ 1);
+    if (U == 1)
+        hipLaunchKernelGGL((k_upkeep<R, 1>), grid, blk, 0, e->stream, a, now, next, c, n, p0, p1, cc);
+    else
+        hipLaunchKernelGGL((k_upkeep<R, 2>), grid, blk, 0, e->stream, a, now, next, c, n, p0, p1, cc);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -1418,7 +1431,7 @@ void mdx_destroy(mdx_engine *e)
                    &e->badj_n,  &e->badj_p,  &e->badj_s, &e->bF,     &e->bT,      &e->bscr,
                    &e->bnscr,   &e->bspecies, &e->bdtab, &e->bttab,  &e->btr4,
                    &e->plpairs, &e->plmask, &e->dmeta,  &e->head,   &e->link,
-                   &e->utot,    &e->usync,  &e->arank,  &e->acount, &e->absum,
+                   &e->utot,    &e->usync,  &e->bucket,  &e->arank,  &e->acount, &e->absum,
                    &e->asorted, &e->aedge,  &e->alab};
     for (Buf *b : bufs)
         dfree(*b);

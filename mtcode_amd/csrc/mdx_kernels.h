@@ -113,9 +113,11 @@ template <class R> struct KArgs {
     unsigned int *dslot;
     // list steps count their force evaluation before it (k_upkeep): 1 there
     int ep_off;
-    // k_upkeep's working arrays: per cell the first particle of its chain plus
-    // one (0: empty; all 0 between builds) and per particle the next one,
+    // k_upkeep's working arrays: per cell the original indices of its first
+    // UP_BUCKET arrivals; the later ones chained per cell: the first of the
+    // chain plus one (0: none; all 0 between builds) and per particle the next;
     // tagged chunk totals of the scan, ticket and phase counters
+    unsigned int *bucket;
     int *head, *link;
     unsigned long long *utot;
     unsigned int *usync;
@@ -2030,7 +2032,10 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_integrate(
 // memory instead.  NB_CAP: 800 (38 KB of LDS, 4 blocks per CU) for sparse
 // systems, 1152 (50 KB, 3 blocks) where an x-row of cells holds many
 // particles (the host picks it from the mean particles per row).
-constexpr int UP_SYNC = 4;     // k_upkeep: ticket counter, then done counts per phase
+// k_upkeep: ticket counter, then done counts per phase, each in a line of its
+// own (the waiting blocks' reads would hold up the others)
+constexpr int UP_LINE = 32, UP_SYNC = 3 * UP_LINE;
+constexpr int UP_BUCKET = 4;   // k_upkeep: arrivals per cell held in its bucket
 constexpr int NB_W = 16;        // own x-rows of a block walked from LDS
 constexpr int NB_CAP_S = 800;   // staged particles per z offset (sparse)
 constexpr int NB_CAP_D = 1152;  // (dense)
@@ -2781,15 +2786,19 @@ __global__ void __launch_bounds__(64) k_call_begin(StepCtl *ctl, unsigned int *d
 // needs an L2 write-back, which made an earlier form of this with fences
 // eight times slower than separate kernels.
 //
-// Binning chains the particles of a cell (head, link) as well as counting
-// them; placing walks a particle's chain and counts the smaller original
-// indices, so the particles of a cell are listed in ascending original index
-// whatever the order of the atomics -- the order the gather's and the list's
-// floating-point sums depend on -- without a sorting pass.
-constexpr int UP_T = 1024;           // threads per block
-constexpr int UP_U = 4;              // particles (cells) per thread and round
-constexpr int UP_CHUNK = UP_T * UP_U; // particles per ticket
-constexpr int UP_MAXTOT = UP_T;      // most chunks of the scan
+// Binning also puts a particle's original index into its cell's bucket (the
+// fifth and later arrivals are chained); placing counts the smaller indices
+// of the cell, so the particles of a cell are listed in ascending original
+// index whatever the order of the atomics -- the order the gather's and the
+// list's floating-point sums depend on -- without a sorting pass.  Bound by the
+// counting atomics and the latency of its phases.  With a chain for every
+// particle (two atomics each), the counters in one line and the waiting blocks
+// reading it without a pause a rebuild took 114 us for 1,048,576 particles in
+// 1,481,544 cells, now 77 (4,096 particles: 26, now 11; 262,144 polymer beads:
+// 50, now 30).
+constexpr int UP_T = 1024;        // threads per block
+constexpr int UP_SCAN = 4 * UP_T; // cells per scan tile
+constexpr int UP_MAXTOT = UP_T;   // most chunks of the scan
 
 template <class T> __device__ __forceinline__ T agent_load(const T *p)
 {
@@ -2824,9 +2833,9 @@ __device__ __forceinline__ int block_scan(int v, int *sh, int &prefix)
 }
 
 // dsl: the drift slots of the current state buffer, dslc: those to clear;
-// cur: that buffer; p0, p1: tickets of a particle phase and of the scan; cc:
-// cells per scan ticket (a multiple of UP_CHUNK)
-template <class R>
+// cur: that buffer; p0, p1: tickets of a particle phase (UP_T * U particles
+// each) and of the scan; cc: cells per scan ticket (a multiple of UP_SCAN)
+template <class R, int U>
 __global__ void __launch_bounds__(UP_T) k_upkeep(KArgs<R> a, const unsigned int *dsl,
                                                  unsigned int *dslc, int cur, int ncells, int p0,
                                                  int p1, int cc)
@@ -2869,15 +2878,16 @@ __global__ void __launch_bounds__(UP_T) k_upkeep(KArgs<R> a, const unsigned int 
         if (phase > 0) {
             const unsigned int want = phase == 1 ? p0 : p1;
             if (tid == 0)
-                while (agent_load(&a.usync[phase]) < want)
-                    __builtin_amdgcn_s_sleep(2);
+                while (agent_load(&a.usync[phase * UP_LINE]) < want)
+                    __builtin_amdgcn_s_sleep(16);
             __syncthreads();
         }
         if (phase == 0) {
-            const int lo = t * UP_CHUNK + tid;
-            int c[UP_U], old[UP_U];
+            const int lo = t * (UP_T * U) + tid;
+            int c[U], r[U];
+            uint32_t id[U];
 #pragma unroll
-            for (int u = 0; u < UP_U; u++) {
+            for (int u = 0; u < U; u++) {
                 const int i = lo + u * UP_T;
                 c[u] = -1;
                 if (i < a.N) {
@@ -2887,87 +2897,98 @@ __global__ void __launch_bounds__(UP_T) k_upkeep(KArgs<R> a, const unsigned int 
                     const int cy = axis_cell(x.y, rp.nc[1], rp.l[1]);
                     const int cz = axis_cell(x.z, rp.nc[2], rp.l[2]);
                     c[u] = rp.coff + cx + rp.nc[0] * (cy + rp.nc[1] * cz);
+                    id[u] = x.id;
                 }
             }
 #pragma unroll
-            for (int u = 0; u < UP_U; u++)
-                if (c[u] >= 0) {
-                    old[u] = atomicExch(&a.head[c[u]], lo + u * UP_T + 1);
-                    atomicAdd(&a.count[c[u]], 1);
-                }
+            for (int u = 0; u < U; u++)
+                if (c[u] >= 0)
+                    r[u] = atomicAdd(&a.count[c[u]], 1);
 #pragma unroll
-            for (int u = 0; u < UP_U; u++)
+            for (int u = 0; u < U; u++)
                 if (c[u] >= 0) {
-                    agent_store(&a.bcell[lo + u * UP_T], c[u]);
-                    agent_store(&a.link[lo + u * UP_T], old[u]);
+                    const int i = lo + u * UP_T;
+                    agent_store(&a.bcell[i], c[u]);
+                    if (r[u] < UP_BUCKET)
+                        agent_store(&a.bucket[(size_t)c[u] * UP_BUCKET + r[u]], id[u]);
+                    else
+                        agent_store(&a.link[i], atomicExch(&a.head[c[u]], i + 1));
                 }
         } else if (phase == 1) {
-            const int k = t - p0, first = k * cc;
+            const int k = t - p0, first = k * cc, last = min(first + cc, ncells);
             int *start = const_cast<int *>(a.start);
+            // four counts of a tile per thread, as two 8-byte loads (the array
+            // is padded to whole tiles)
+            auto load4 = [&](int b, int v[4]) -> int {
+                const unsigned long long *p =
+                    reinterpret_cast<const unsigned long long *>(a.count + b) + 2 * tid;
+                const unsigned long long w0 = agent_load(p), w1 = agent_load(p + 1);
+                v[0] = (int)(unsigned int)w0;
+                v[1] = (int)(w0 >> 32);
+                v[2] = (int)(unsigned int)w1;
+                v[3] = (int)(w1 >> 32);
+                return v[0] + v[1] + v[2] + v[3];
+            };
             // the chunk's total, then the totals before it, then its starts
-            int sum = 0;
-            for (int b = first; b < min(first + cc, ncells); b += UP_CHUNK)
-#pragma unroll
-                for (int u = 0; u < UP_U; u++) {
-                    const int c = b + tid * UP_U + u;
-                    sum += c < ncells ? agent_load(&a.count[c]) : 0;
-                }
-            int run;
+            // (a chunk of one tile keeps its counts)
+            int v[4], run, sum = 0;
+            for (int b = first; b < last; b += UP_SCAN)
+                sum += load4(b, v);
             const int total = block_scan(sum, sh, run);
             if (tid == 0)
                 agent_store(&a.utot[k], ((unsigned long long)tag << 32) | (unsigned int)total);
             int before = 0;
             if (tid < k) {
-                unsigned long long v;
-                while ((unsigned int)((v = agent_load(&a.utot[tid])) >> 32) != tag)
-                    __builtin_amdgcn_s_sleep(1);
-                before = (int)(unsigned int)v;
+                unsigned long long w;
+                while ((unsigned int)((w = agent_load(&a.utot[tid])) >> 32) != tag)
+                    __builtin_amdgcn_s_sleep(8);
+                before = (int)(unsigned int)w;
             }
+            int mine = run;
             int base = block_scan(before, sh, run);
-            for (int b = first; b < min(first + cc, ncells); b += UP_CHUNK) {
-                int v[UP_U], s = 0;
-#pragma unroll
-                for (int u = 0; u < UP_U; u++) {
-                    const int c = b + tid * UP_U + u;
-                    v[u] = c < ncells ? agent_load(&a.count[c]) : 0;
-                    s += v[u];
-                }
-                const int all = block_scan(s, sh, run);
+            for (int b = first; b < last; b += UP_SCAN) {
+                int all = total;
+                run = mine;
+                if (cc != UP_SCAN)
+                    all = block_scan(load4(b, v), sh, run);
                 run += base;
-#pragma unroll
-                for (int u = 0; u < UP_U; u++) {
-                    const int c = b + tid * UP_U + u;
-                    if (c < ncells) {
-                        agent_store(&start[c], run);
-                        a.count[c] = 0;
-                    }
-                    run += v[u];
-                }
+                const int s0 = run, s1 = s0 + v[0], s2 = s1 + v[1], s3 = s2 + v[2];
+                unsigned long long *o = reinterpret_cast<unsigned long long *>(start + b) + 2 * tid;
+                agent_store(o, ((unsigned long long)(unsigned int)s1 << 32) | (unsigned int)s0);
+                agent_store(o + 1, ((unsigned long long)(unsigned int)s3 << 32) | (unsigned int)s2);
+                reinterpret_cast<int4 *>(a.count + b)[tid] = make_int4(0, 0, 0, 0);
                 base += all;
             }
-            if (k == p1 - 1 && tid == 0)
-                start[ncells] = base;
         } else {
-            const int lo = (t - p0 - p1) * UP_CHUNK + tid;
-            int c[UP_U], j[UP_U], at[UP_U];
+            const int lo = (t - p0 - p1) * (UP_T * U) + tid;
+            int c[U], at[U], m[U];
 #pragma unroll
-            for (int u = 0; u < UP_U; u++)
+            for (int u = 0; u < U; u++)
                 c[u] = lo + u * UP_T < a.N ? agent_load(&a.bcell[lo + u * UP_T]) : -1;
 #pragma unroll
-            for (int u = 0; u < UP_U; u++)
+            for (int u = 0; u < U; u++)
                 if (c[u] >= 0) {
-                    j[u] = agent_load(&a.head[c[u]]);
                     at[u] = agent_load(&a.start[c[u]]);
+                    m[u] = agent_load(&a.start[c[u] + 1]) - at[u];
                 }
 #pragma unroll
-            for (int u = 0; u < UP_U; u++)
+            for (int u = 0; u < U; u++)
                 if (c[u] >= 0) {
                     const int i = lo + u * UP_T;
-                    const uint32_t id = a.X[i].id;
-                    for (int q = j[u]; q != 0;) {
-                        if (q - 1 != i)
-                            at[u] += a.X[q - 1].id < id ? 1 : 0;
-                        q = agent_load(&a.link[q - 1]);
+                    if (m[u] > 1) {
+                        const uint32_t id = a.X[i].id;
+                        const unsigned int *bk = a.bucket + (size_t)c[u] * UP_BUCKET;
+                        unsigned int w[UP_BUCKET];
+#pragma unroll
+                        for (int q = 0; q < UP_BUCKET; q++)
+                            w[q] = agent_load(bk + q);
+#pragma unroll
+                        for (int q = 0; q < UP_BUCKET; q++)
+                            at[u] += q < m[u] && w[q] < id ? 1 : 0;
+                        if (m[u] > UP_BUCKET)
+                            for (int q = agent_load(&a.head[c[u]]); q != 0;
+                                 q = agent_load(&a.link[q - 1]))
+                                at[u] += a.X[q - 1].id < id ? 1 : 0;
                     }
                     const_cast<int *>(a.list)[at[u]] = i;
                 }
@@ -2976,7 +2997,7 @@ __global__ void __launch_bounds__(UP_T) k_upkeep(KArgs<R> a, const unsigned int 
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tid == 0 && phase < 2)
-            atomicAdd(&a.usync[phase + 1], 1u);
+            atomicAdd(&a.usync[(phase + 1) * UP_LINE], 1u);
     }
 }
 
