@@ -983,26 +983,46 @@ template <class R> static int upkeep(mdx_engine *e)
 }
 
 // neighbour list of the current slots from the cell list just built
-template <class R> static int build_list(mdx_engine *e, const int *cells, int gated)
+// (exact: only pairs within the list radii in FP64)
+template <class R>
+static int build_list(mdx_engine *e, const int *cells, int gated, bool exact = false)
 {
     KArgs<R> a = make_args<R>(e);
     a.lmode = 1;
     // the larger LDS staging where an x-row of cells holds many particles
     // (about 3 + 256 / row rows of particles staged per z offset of a block)
     long long rows = 0;
-    for (const DevRep &r : e->reps)
+    double lmax = 0;
+    for (const DevRep &r : e->reps) {
         rows += (long long)r.nc[1] * r.nc[2];
+        lmax = std::max(lmax, std::max(r.l[0], std::max(r.l[1], r.l[2])));
+    }
     const double per_row = rows > 0 ? (double)e->N / (double)rows : 0.0;
     const bool dense =
         e->nb_dense >= 0
             ? e->nb_dense != 0
             : per_row > 0 && (std::ceil(256.0 / per_row) + 3.0) * per_row > 0.9 * NB_CAP_S;
-    if (dense)
-        hipLaunchKernelGGL((k_nbuild<R, NB_CAP_D>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a,
-                           cells, gated);
+    // error of an FP32 squared distance near the list radius rl: coordinates
+    // and box edges are off by up to 2^-24 L each, so a component by 3 of
+    // these, the square by 2 sqrt(3) rl times that, and 4 roundings of rl^2:
+    // below 11 * 2^-24 (L + rl) rl.  Nearly three times that is added
+    const double rl = std::sqrt(a.rl2), slack = 32 * 5.97e-8 * (lmax + rl) * rl;
+    const float rl2f = (float)(a.rl2 + slack), rl2wf = (float)(a.rl2w + slack);
+    const dim3 blk(256);
+#define NBUILD(CAP, LP)                                                                          \
+    hipLaunchKernelGGL((k_nbuild<R, CAP, LP>), dim3(nblk(e->N, 256 / LP)), blk, 0, e->stream, a,  \
+                       cells, gated, exact ? 1 : 0, rl2f, rl2wf)
+    // four lanes per position while the longest lane bounds the build (us per
+    // step with 4 / 1 lanes, tetrahedral and condensate, mixed: 4,000 particles
+    // 21.7 / 24.0 and 20.5 / 23.1, 70,000 47.9 / 50.1 and 36.5 / 38.0, 130,000
+    // 55.1 / 54.7 and 43.5 / 42.6)
+    if (e->N <= 100000)
+        NBUILD(NB_CAP_S, 4);
+    else if (dense)
+        NBUILD(NB_CAP_D, 1);
     else
-        hipLaunchKernelGGL((k_nbuild<R, NB_CAP_S>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a,
-                           cells, gated);
+        NBUILD(NB_CAP_S, 1);
+#undef NBUILD
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -2851,7 +2871,7 @@ static int list_pairs_t(mdx_engine *e, int *ij, long long cap, long long *npairs
         return rc;
     if (!e->counted && (rc = count_current<R>(e)))
         return rc;
-    if ((rc = finish_bins(e)) || (rc = build_list<R>(e, (const int *)e->cell[e->cur].p, 0)))
+    if ((rc = finish_bins(e)) || (rc = build_list<R>(e, (const int *)e->cell[e->cur].p, 0, true)))
         return rc;
     e->counted = false;
     e->binned = true;

@@ -2016,21 +2016,28 @@ template <class R, int MODE> __global__ void __launch_bounds__(256) k_integrate(
 // x, x + 1 of the row), written to nbr[k * N + slot] with the count in nn;
 // the compacted walk lays the entries out per block afterwards (fresh).
 // gated: only when a rebuild was requested.
-// One thread per cell-list position: a block's particles then lie in a few
-// consecutive x-rows of cells (the list is in cell order).  The block first
+// LP threads per cell-list position (1; 4 for small systems, where the longest
+// lane bounds the build): a block's particles then lie in a few consecutive
+// x-rows of cells (the list is in cell order).  The block first
 // finds, for each z offset (one wave each), the distinct neighbour rows of
 // its rows and loads their cell offsets into LDS; then, one z offset at a
-// time, it stages those rows' particles (position record and slot, read with
-// coalesced loads from the list) and walks them there.  Each staged row
-// holds its last cell, the row, then its first cell again, so that the three
-// cells about any x -- across the periodic seam too -- are one contiguous
-// run.  The walk first marks the candidates within the list radius in a bit
-// mask (a distance per candidate, no other work), then takes the marked ones
-// in order.  A block whose particles span more than NB_W rows or two
+// time, it stages those rows' particles (FP32 position and original index in
+// 16 B, slot, type; read with coalesced loads from the list) and walks them
+// there.  Each staged row holds its last cell, the row, then its first cell
+// again, so that the three cells about any x -- across the periodic seam too
+// -- are one contiguous run.  The walk first marks the candidates within the
+// list radius in a bit mask (a distance per candidate, no other work), then
+// takes the marked ones in order.  The marks are FP32 distances against the
+// radius plus a bound on their error (rl2f, rl2wf: the host's), so a list holds
+// every pair within the radius and may hold a few just beyond it, which add
+// nothing to any sum (the walk's own FP64 cut-offs are shorter by the skin);
+// exact: those are left out again by their FP64 distance (mdx_list_pairs).
+// With FP64 records staged (32 B, two LDS reads per candidate, 38 KB) the walk
+// was bound by LDS reads and by 4 blocks per CU.  A block whose particles span more than NB_W rows or two
 // replicas, a grid with fewer than 3 cells on a side, and a z offset whose
 // rows hold more than NB_CAP particles or NB_ROWCAP cell offsets walk global
-// memory instead.  NB_CAP: 800 (38 KB of LDS, 4 blocks per CU) for sparse
-// systems, 1152 (50 KB, 3 blocks) where an x-row of cells holds many
+// memory instead.  NB_CAP: 800 (26 KB of LDS, 6 blocks per CU) for sparse
+// systems, 1152 (33 KB, 4 blocks) where an x-row of cells holds many
 // particles (the host picks it from the mean particles per row).
 // k_upkeep: ticket counter, then done counts per phase, each in a line of its
 // own (the waiting blocks' reads would hold up the others)
@@ -2070,13 +2077,19 @@ __device__ __forceinline__ void row_ranges(const T *off, int n0, int cx, int &r0
     }
 }
 
-template <class R, int NB_CAP>
-__global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, int gated)
+// The sparse one-lane form is held to 80 VGPRs (6 waves per SIMD, no spill: 120
+// -> 106 us).  Measured, a rebuild's list: 1,048,576-particle condensate 145
+// (FP64 records) -> 106 us, 64 replicas (298,897) 98 -> 76, 262,144 polymer
+// beads 68 -> 61, 4,096 particles 42 -> 19 (four lanes per position).
+template <class R, int NB_CAP, int LP>
+__global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1) k_nbuild(KArgs<R> a, const int *cells, int gated, int exact,
+                                                float rl2f, float rl2wf)
 {
     if (gated && !a.ctl->rebuild)
         return;
-    __shared__ PosRec lpos[NB_CAP];
+    __shared__ float4 lpos[NB_CAP]; // x, y, z, original index (bits)
     __shared__ int lslot[NB_CAP];
+    __shared__ unsigned char ltype[NB_CAP];
     // per z offset p: n0 + 1 cell offsets per staged row, relative to the
     // row's first list position hk0
     __shared__ unsigned short rowoff[3][NB_ROWCAP];
@@ -2096,9 +2109,10 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
     // k_upkeep's counters and chains as it expects them next time
     if (blockIdx.x == 0 && tid < UP_SYNC)
         a.usync[tid] = 0u;
-    const int p0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x;
-    const int pos = p0 + tid;
-    const int plast = min(p0 + (int)blockDim.x, a.N) - 1;
+    constexpr int PB = 256 / LP; // positions per block
+    const int p0 = xcd_block(blockIdx.x, gridDim.x) * PB;
+    const int pos = p0 + tid / LP, sub = tid % LP;
+    const int plast = min(p0 + PB, a.N) - 1;
     const bool live = pos <= plast;
     int s = 0, c = 0;
     PosRec xi;
@@ -2106,8 +2120,10 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
         s = a.list[pos];
         xi = a.X[s];
         c = cells[s];
-        a.bcell[s] = c;
-        a.head[c] = 0;
+        if (sub == 0) {
+            a.bcell[s] = c;
+            a.head[c] = 0;
+        }
         if (pos == p0) {
             ends[0] = (int)(xi.meta >> 8);
             ends[1] = c;
@@ -2148,12 +2164,11 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
         ti = xi.meta & 255;
     }
     // the pair's types carry an active patch row
-    auto patch_active = [&](const PosRec &xj) -> bool {
-        const int tj = xj.meta & 255;
-        if (!(a.has_patches && a.np[ti] > 0 && a.np[tj] > 0))
+    auto patch_active = [&](uint32_t idj, int tj) -> bool {
+        if (!a.has_patches)
             return false;
         int ta, tc;
-        patch_roles(xi.id, ti, xj.id, tj, ta, tc);
+        patch_roles(xi.id, ti, idj, tj, ta, tc);
         return (a.active_mask >> (ta * MAXT + tc)) & 1ull;
     };
     // plain: no candidate can be a periodic image (the cell is off the box
@@ -2171,27 +2186,28 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
         }
         return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
     };
-    // a candidate within the list radius (r2 < rl2): listed unless beyond
-    // the WCA reach without patch terms, or an exclusion without them
-    auto take = [&](const PosRec &xj, int j, double r2) {
-        if (!(r2 < a.rl2w) && !patch_active(xj))
-            return;
+    // a candidate within the list radius: listed unless beyond the WCA reach
+    // (far) without patch terms, or an exclusion without them
+    auto listed = [&](uint32_t idj, int tj, bool far) -> bool {
+        if (far && !patch_active(idj, tj))
+            return false;
         bool ex = false;
         for (int e = exc0; e < exc1; e++)
-            ex |= (uint32_t)a.exc_j[e] == xj.id;
+            ex |= (uint32_t)a.exc_j[e] == idj;
         if (ex) {
-            if (!patch_active(xj))
-                return;
+            if (!patch_active(idj, tj))
+                return false;
             kept_excluded = true;
         }
-        if (n < a.kmax)
-            a.nbrw[(size_t)n * a.N + s] = j;
-        n++;
+        return true;
     };
     auto consider = [&](const PosRec &xj, int j) {
         const double r2 = dist2(xj);
-        if (r2 < a.rl2)
-            take(xj, j, r2);
+        if (r2 < a.rl2 && listed(xj.id, (int)(xj.meta & 255u), !(r2 < a.rl2w))) {
+            if (n < a.kmax)
+                a.nbrw[(size_t)n * a.N + s] = j;
+            n++;
+        }
     };
     auto global_range = [&](int r0, int r1) {
         for (int k = r0; k < r1; k++) {
@@ -2202,8 +2218,9 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
     };
 
     if (binfo[0] < 0) {
-        // the 27 cells from global memory, in the same order
-        if (live) {
+        // the 27 cells from global memory, in the same order (the first of a
+        // position's lanes)
+        if (live && sub == 0) {
             const int cl = c - rp.coff;
             const int n0 = rp.nc[0], n1 = rp.nc[1], n2 = rp.nc[2];
             const int cx = cl % n0, cy = (cl / n0) % n1, cz = cl / (n0 * n1);
@@ -2231,6 +2248,12 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
         const int cy = (cc / n0) % n1, cz = cc / (n0 * n1);
         plain = !a.periodic || (n0 >= 5 && n1 >= 5 && n2 >= 5 && cx >= 1 && cx <= n0 - 2 &&
                                 cy >= 1 && cy <= n1 - 2 && cz >= 1 && cz <= n2 - 2);
+        const float xf[3] = {(float)xi.x, (float)xi.y, (float)xi.z};
+        float lf[3], hf[3]; // box edges and their halves (walls: never reached)
+        for (int k = 0; k < 3; k++) {
+            lf[k] = (float)rb.l[k];
+            hf[k] = a.periodic ? 0.5f * lf[k] : 3.0e38f;
+        }
         const int wv = tid >> 6, lane = tid & 63;
         // wave p (z offset p - 1): the candidate rows, own row rf + m / 3
         // moved by m % 3 - 1 in y and by p - 1 in z; the distinct ones are
@@ -2327,8 +2350,11 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
                     int o = f - hoff[p][lo];
                     o = o < cl ? off[n0 - 1] + o : (o < cl + cr ? o - cl : o - cl - cr);
                     const int j = a.list[hk0[p][lo] + o];
+                    const PosRec xj = a.X[j];
                     lslot[f] = j;
-                    lpos[f] = a.X[j];
+                    ltype[f] = (unsigned char)xj.meta;
+                    lpos[f] = make_float4((float)xj.x, (float)xj.y, (float)xj.z,
+                                          __uint_as_float(xj.id));
                 }
             __syncthreads();
             if (live && staged) {
@@ -2346,26 +2372,60 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
                     tot += b1 - b0;
                     cum[dy] = tot;
                 }
-                // marks, 64 candidates at a time, then the marked ones in order
+                auto at = [&](int t) -> int {
+                    return t < cum[0] ? qs[0] + t
+                                      : (t < cum[1] ? qs[1] + t - cum[0] : qs[2] + t - cum[1]);
+                };
+                auto dist2f = [&](const float4 &v) -> float {
+                    float d[3] = {xf[0] - v.x, xf[1] - v.y, xf[2] - v.z};
+                    if (!plain)
+                        for (int k = 0; k < 3; k++)
+                            d[k] -= d[k] > hf[k] ? lf[k] : (d[k] < -hf[k] ? -lf[k] : 0.f);
+                    return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+                };
+                // 64 candidates at a time: marks (a lane takes two per round,
+                // their reads overlap; several lanes of a position take
+                // candidates in turn), then of the marked ones those that are
+                // listed, then their places in order
                 for (int t0 = 0; t0 < tot; t0 += 64) {
                     const int te = min(tot, t0 + 64);
-                    unsigned long long hit = 0ull;
-                    for (int t = t0; t < te; t++) {
-                        const int q = t < cum[0] ? qs[0] + t
-                                                 : (t < cum[1] ? qs[1] + t - cum[0] : qs[2] + t - cum[1]);
-                        const PosRec &xj = lpos[q];
-                        if (xj.id != xi.id && dist2(xj) < a.rl2)
+                    unsigned long long hit = 0ull, keep = 0ull;
+                    for (int t = t0 + sub; t < te; t += 2 * LP) {
+                        const bool two = t + LP < te;
+                        const float4 v0 = lpos[at(t)], v1 = lpos[at(two ? t + LP : t)];
+                        if (dist2f(v0) < rl2f && __float_as_uint(v0.w) != xi.id)
                             hit |= 1ull << (t - t0);
+                        if (two && dist2f(v1) < rl2f && __float_as_uint(v1.w) != xi.id)
+                            hit |= 1ull << (t + LP - t0);
                     }
                     while (hit) {
-                        const int t = t0 + __builtin_ctzll(hit);
+                        const int b = __builtin_ctzll(hit);
                         hit &= hit - 1ull;
-                        const int q = t < cum[0] ? qs[0] + t
-                                                 : (t < cum[1] ? qs[1] + t - cum[0] : qs[2] + t - cum[1]);
-                        take(lpos[q], lslot[q], dist2(lpos[q]));
+                        const int q = at(t0 + b);
+                        const float4 v = lpos[q];
+                        bool far = !(dist2f(v) < rl2wf);
+                        if (exact) {
+                            const double r2 = dist2(a.X[lslot[q]]);
+                            if (!(r2 < a.rl2))
+                                continue;
+                            far = !(r2 < a.rl2w);
+                        }
+                        if (listed(__float_as_uint(v.w), ltype[q], far))
+                            keep |= 1ull << b;
                     }
+                    unsigned long long all = keep;
+                    for (int o = 1; o < LP; o <<= 1)
+                        all |= __shfl_xor(all, o);
+                    while (keep) {
+                        const int b = __builtin_ctzll(keep);
+                        keep &= keep - 1ull;
+                        const int k = n + __popcll(all & ((1ull << b) - 1ull));
+                        if (k < a.kmax)
+                            a.nbrw[(size_t)k * a.N + s] = lslot[at(t0 + b)];
+                    }
+                    n += __popcll(all);
                 }
-            } else if (live) {
+            } else if (live && sub == 0) {
                 for (int dy = 0; dy < 3; dy++) {
                     int r0, r1, r2, r3;
                     row_ranges(a.start + crow[p][3 * ro + dy], n0, cx, r0, r1, r2, r3);
@@ -2373,11 +2433,16 @@ __global__ void __launch_bounds__(256) k_nbuild(KArgs<R> a, const int *cells, in
                     global_range(r2, r3);
                 }
             }
+            if (LP > 1 && !staged)
+                n = __shfl(n, lane - lane % LP);
             __syncthreads();
         }
     }
-    if (live)
-        a.nn[s] = n | (kept_excluded ? LIST_EXC : 0);
+    int ke = kept_excluded ? 1 : 0;
+    for (int o = 1; o < LP; o <<= 1)
+        ke |= __shfl_xor(ke, o);
+    if (live && sub == 0)
+        a.nn[s] = n | (ke ? LIST_EXC : 0);
 }
 
 // ------------------------------------------------------- LDS-staged tiles
