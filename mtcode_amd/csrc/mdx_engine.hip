@@ -186,6 +186,14 @@ struct mdx_engine {
     Buf dslot;           // drift maxima slots, NDSLOT per state buffer
     Buf bucket, head, link, utot, usync; // k_upkeep
     Buf arank, acount, absum;    // the analysis grids' cell lists
+    // slot tables of the topology in list steps (k_topo_slots): usable while
+    // no particle has more than TOPO_B bonds or TOPO_A angles; stale after a
+    // change of the topology
+    Buf tbond, tang, tact;
+    int max_bonds = 0, max_angles = 0;
+    int bond_uni = 0, ang_uni = 0;
+    double ubk = 0, ubr0 = 0, uak = 0, uat0 = 0;
+    bool topo_stale = true;
     Buf asorted, aedge, alab;    // positions in cell order, bin edges, cluster labels
     hipEvent_t prof_mid = nullptr;  // recorded between walk and finish while profiling
     hipEvent_t prof_mid2 = nullptr; // recorded between patch and integrate while profiling
@@ -714,6 +722,17 @@ template <class R> static int bin_current(mdx_engine *e)
 template <class R, int MODE>
 static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode);
 
+template <class R> static void topo_args(const mdx_engine *e, KArgs<R> &a);
+
+template <class R, int MODE> static void launch_integrate(mdx_engine *e, const KArgs<R> &a)
+{
+    // without topology the kernel carries no code for it (98 VGPRs with)
+    if (MODE == M_CONS || e->nbonds || e->nangles || e->has_active)
+        hipLaunchKernelGGL((k_integrate<R, MODE, true>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
+    else
+        hipLaunchKernelGGL((k_integrate<R, MODE, false>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
+}
+
 // split form of a force evaluation: walk, patch kernel, integrator
 template <class R, int MODE>
 static int launch_split(mdx_engine *e, KArgs<R> &a, int lmode, bool bead_list)
@@ -790,7 +809,7 @@ static int launch_split(mdx_engine *e, KArgs<R> &a, int lmode, bool bead_list)
     if (e->prof_mid2)
         HIPCHK(hipEventRecord(e->prof_mid2, e->stream));
     if (bead_list || e->use_compact) {
-        hipLaunchKernelGGL((k_integrate<R, MODE>), grid, blk, 0, e->stream, a);
+        launch_integrate<R, MODE>(e, a);
     } else if constexpr (patches) {
         hipLaunchKernelGGL((k_finish<R, MODE>), grid, blk, 0, e->stream, a);
     }
@@ -809,6 +828,7 @@ static int launch_gather(mdx_engine *e, const double *noise_dev, int lmode = 0)
     a.noise = noise_dev;
     a.lmode = lmode;
     a.ep_off = lmode ? 1 : 0; // (list steps: k_upkeep has counted the evaluation)
+    topo_args(e, a);
     // split form: patch systems, and list steps of the bead integrator (walk,
     // then the integrator kernel; no patch kernel)
     const bool bead_list = MODE == M_BEAD && lmode && e->use_walkc;
@@ -916,6 +936,43 @@ static void call_begin(mdx_engine *e)
 {
     hipLaunchKernelGGL(k_call_begin, dim3(1), dim3(NDSLOT), 0, e->stream, (StepCtl *)e->ctl.p,
                        (unsigned int *)e->dslot.p, e->cur, e->integ == MDX_INTEG_ROTOR ? 1 : 0);
+}
+
+// the topology's slot tables for the list steps from the current slots
+template <class R> static int topo_tables(mdx_engine *e)
+{
+    const bool any = e->nbonds || e->nangles || e->has_active;
+    if (!any || e->max_bonds > TOPO_B || e->max_angles > TOPO_A)
+        return MDX_OK;
+    int rc;
+    if ((e->nbonds && (rc = dalloc(e, e->tbond, 16 * (size_t)e->N))) ||
+        (e->nangles && (rc = dalloc(e, e->tang, 32 * (size_t)e->N))) ||
+        (e->has_active && (rc = dalloc(e, e->tact, 8 * (size_t)e->N))))
+        return rc;
+    hipLaunchKernelGGL(k_topo_slots<R>, dim3(nblk(e->N)), dim3(256), 0, e->stream, make_args<R>(e),
+                       e->nbonds ? (int4 *)e->tbond.p : nullptr,
+                       e->nangles ? (int4 *)e->tang.p : nullptr,
+                       e->has_active ? (int2 *)e->tact.p : nullptr);
+    HIPCHK(hipGetLastError());
+    e->topo_stale = false;
+    return MDX_OK;
+}
+
+// the list steps' view of them (never a stale table)
+template <class R> static void topo_args(const mdx_engine *e, KArgs<R> &a)
+{
+    if (!a.lmode || e->topo_stale)
+        return;
+    a.ell = 1;
+    a.tbond = e->nbonds ? (const int4 *)e->tbond.p : nullptr;
+    a.tang = e->nangles ? (const int4 *)e->tang.p : nullptr;
+    a.tact = e->has_active ? (const int2 *)e->tact.p : nullptr;
+    a.bond_uni = e->bond_uni;
+    a.ang_uni = e->ang_uni;
+    a.ubk = e->ubk;
+    a.ubr0 = e->ubr0;
+    a.uak = e->uak;
+    a.uat0 = e->uat0;
 }
 
 template <class R> static int do_prime(mdx_engine *e, const double *noise0)
@@ -1062,6 +1119,7 @@ template <class R, int MODE> static int list_step_graph(mdx_engine *e, int steps
 {
     KArgs<R> a = make_args<R>(e);
     a.lmode = 1;
+    topo_args(e, a);
     // the arguments, the grid and the launch-form switches (which kernels
     // the step launches)
     const int form[7] = {e->ncells,      e->N,         e->use_split, e->use_compact,
@@ -1163,6 +1221,7 @@ static int enqueue_some(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, 
             HIPCHK(hipMemcpyAsync(e->slot[e->cur ^ 1].p, e->slot[e->cur].p, 4 * (size_t)e->N,
                                   hipMemcpyDeviceToDevice, e->stream));
             e->list_valid = true;
+            e->topo_stale = true; // (the slots are new)
             e->since_resort = 0;
             e->binned = MODE == M_BEAD;
         } else {
@@ -1170,6 +1229,8 @@ static int enqueue_some(mdx_engine *e, const double *nd, hipEvent_t *ev, int s, 
         }
         e->counted = false;
     } else {
+        if (e->topo_stale && (rc = topo_tables<R>(e)))
+            return rc;
         // replayed from a captured graph once an eager list step has run
         // with the same launch arguments (engine noise, not profiling)
         const bool graph = e->use_graph && !ev && !nd && MODE != M_STEP && e->list_eager;
@@ -1452,7 +1513,7 @@ void mdx_destroy(mdx_engine *e)
                    &e->bnscr,   &e->bspecies, &e->bdtab, &e->bttab,  &e->btr4,
                    &e->plpairs, &e->plmask, &e->dmeta,  &e->head,   &e->link,
                    &e->utot,    &e->usync,  &e->bucket,  &e->arank,  &e->acount, &e->absum,
-                   &e->asorted, &e->aedge,  &e->alab};
+                   &e->asorted, &e->aedge,  &e->alab,   &e->tbond,  &e->tang,   &e->tact};
     for (Buf *b : bufs)
         dfree(*b);
     for (hipEvent_t ev : e->pin_ev)
@@ -1769,6 +1830,23 @@ static void csr(int N, const std::vector<std::pair<int, int>> &ent, std::vector<
         val[cur[p.first]++] = p.second;
 }
 
+// the longest row of a CSR
+static int max_row(const std::vector<int> &off)
+{
+    int m = 0;
+    for (size_t i = 0; i + 1 < off.size(); i++)
+        m = std::max(m, off[i + 1] - off[i]);
+    return m;
+}
+
+static int all_equal(const double *v, long long n)
+{
+    for (long long i = 1; i < n; i++)
+        if (!(v[i] == v[0]))
+            return 0;
+    return n > 0;
+}
+
 static int check_same_replica(mdx_engine *e, const int *idx, int n, long long row)
 {
     int r0 = -1;
@@ -1826,6 +1904,11 @@ int mdx_set_bonds(mdx_engine *e, long long nbonds, const int *ij, const double *
         return rc;
     e->nbonds = nbonds;
     e->bond_kind = kind;
+    e->max_bonds = max_row(off);
+    e->bond_uni = all_equal(k, nbonds) && all_equal(r0, nbonds);
+    e->ubk = nbonds ? k[0] : 0.0;
+    e->ubr0 = nbonds ? r0[0] : 0.0;
+    e->topo_stale = true;
     return MDX_OK;
 }
 
@@ -1859,6 +1942,11 @@ int mdx_set_angles(mdx_engine *e, long long nangles, const int *ijk, const doubl
         return rc;
     e->nangles = nangles;
     e->ang_form = form;
+    e->max_angles = max_row(off);
+    e->ang_uni = all_equal(k, nangles) && all_equal(theta0, nangles);
+    e->uak = nangles ? k[0] : 0.0;
+    e->uat0 = nangles ? theta0[0] : 0.0;
+    e->topo_stale = true;
     return MDX_OK;
 }
 
@@ -1901,6 +1989,7 @@ int mdx_set_active(mdx_engine *e, double fa, const int *prev, const int *next)
         return rc;
     e->fa = fa;
     e->has_active = 1;
+    e->topo_stale = true;
     return MDX_OK;
 }
 
@@ -1923,6 +2012,7 @@ int mdx_clear_interactions(mdx_engine *e, int terms)
         e->nexcl = 0;
     if (terms & MDX_TERM_ACTIVE)
         e->has_active = 0;
+    e->topo_stale = true;
     e->grid_dirty = true;
     return MDX_OK;
 }
@@ -2457,6 +2547,7 @@ static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode)
     a.noise = noise_dev;
     a.lmode = lmode;
     a.ep_off = lmode ? 1 : 0; // (list steps: k_upkeep has counted the evaluation)
+    topo_args(e, a);
     const bool list_walk = lmode && e->use_walkc;
     a.pcap = list_walk ? std::max(PMAXG, e->kmax) : PMAXG;
     int rc;
@@ -2504,7 +2595,7 @@ static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode)
     a.bF = (const double *)e->bF.p;
     a.bT = (const double *)e->bT.p;
     a.bncand = (const int *)e->ncand.p;
-    hipLaunchKernelGGL((k_integrate<R, MODE>), dim3(nblk(e->N)), dim3(256), 0, e->stream, a);
+    launch_integrate<R, MODE>(e, a);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
