@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstddef>
@@ -62,11 +63,11 @@ struct Buf {
     size_t bytes = 0;
 };
 
-// device-to-host copies (fetch): up to FETCH_THREADS host threads, each with
-// two pinned slots of at most FETCH_CHUNK bytes
-constexpr int FETCH_THREADS = 4;
+// device-to-host copies (fetch): FETCH_SLOTS pinned slots of at most
+// FETCH_CHUNK bytes, emptied by FETCH_THREADS host threads
+constexpr int FETCH_THREADS = 4, FETCH_SLOTS = 8;
 constexpr size_t FETCH_CHUNK = (size_t)4 << 20;
-constexpr size_t FETCH_SMALL = (size_t)2 << 20; // one slot, one thread, up to here
+constexpr size_t FETCH_SMALL = (size_t)8 << 20; // one slot, no threads, up to here
 // host-to-device copies through the pinned slot up to here (64 KB: 10 us
 // against 32 us pageable; from 128 KB on the two are equal)
 constexpr size_t UPLOAD_PINNED = (size_t)128 << 10;
@@ -163,10 +164,10 @@ struct mdx_engine {
     Buf exc_off, exc_j, act_prev, act_next;
     Buf noise, ctl, partial, tmpd, tmpi, tmpi2, tmpi3, tmpll, tmpx;
     // pinned staging of the device-to-host copies (fetch): at most
-    // 2 FETCH_THREADS FETCH_CHUNK = 32 MiB, given back with the engine
+    // FETCH_SLOTS FETCH_CHUNK = 32 MiB, given back with the engine
     char *pin = nullptr;
     size_t pin_bytes = 0;
-    hipEvent_t pin_ev[2 * FETCH_THREADS] = {};
+    hipEvent_t pin_ev[FETCH_SLOTS] = {};
     Buf dmeta; // meta by original index (uploaded when it changed)
     bool meta_dirty = true;
     Buf Fw, ncand, cand, Tp; // split walk -> (patch ->) finish
@@ -330,14 +331,17 @@ template <class T> static int upload(mdx_engine *e, Buf &b, const T *h, size_t n
 // through the slots 11.3 ms with 1 thread, 6.2 with 2, 4.0 with 4, 3.8 with
 // 8.  Up to FETCH_SMALL bytes one slot, no threads and no events, and one copy
 // where the caller says that the device arrays follow each other in one
-// allocation: a pageable copy costs 7 to 20 us of its own (64 KB: 34 us
-// against 10, 600 KB in two arrays: 39 against 32).
-static int fetch(mdx_engine *e, const Span *sp, int n, bool joined = false)
+// allocation (`meanwhile` is called once the copies are queued): a pageable copy costs 7 to 20 us of its own (64 KB: 34 us
+// against 10, 600 KB in two arrays: 39 against 32).  Starting the threads
+// costs 60 to 150 us (4.6 MB through them took 375 us, one slot 245).
+template <class W>
+static int fetch(mdx_engine *e, const Span *sp, int n, bool joined, W &&meanwhile)
 {
     size_t total = 0;
     for (int k = 0; k < n; k++)
         total += sp[k].bytes;
     if (total == 0) {
+        meanwhile();
         HIPCHK(hipStreamSynchronize(e->stream));
         return MDX_OK;
     }
@@ -353,6 +357,7 @@ static int fetch(mdx_engine *e, const Span *sp, int n, bool joined = false)
                                       e->stream));
             off += len;
         }
+        meanwhile();
         HIPCHK(hipStreamSynchronize(e->stream));
         off = 0;
         for (int k = 0; k < n; k++) {
@@ -362,13 +367,10 @@ static int fetch(mdx_engine *e, const Span *sp, int n, bool joined = false)
         }
         return MDX_OK;
     }
-    // slots sized so that every thread has a few
-    const int T = total < 4 * FETCH_SMALL ? 2 : FETCH_THREADS;
-    const size_t C =
-        std::min(FETCH_CHUNK, std::max(FETCH_CHUNK_MIN, (total / (4 * T) + 4095) & ~(size_t)4095));
-    if ((rc = pin_reserve(e, 2 * T * C)))
+    const size_t C = std::min(FETCH_CHUNK, std::max(FETCH_CHUNK_MIN, (total / 16 + 4095) & ~(size_t)4095));
+    if ((rc = pin_reserve(e, FETCH_SLOTS * C)))
         return rc;
-    for (int k = 0; k < 2 * T; k++)
+    for (int k = 0; k < FETCH_SLOTS; k++)
         if (!e->pin_ev[k])
             HIPCHK(hipEventCreateWithFlags(&e->pin_ev[k], hipEventDisableTiming));
     // piece c of all spans, C bytes at a time (a piece ends with its span)
@@ -383,55 +385,89 @@ static int fetch(mdx_engine *e, const Span *sp, int n, bool joined = false)
         d = (const char *)sp[k].dev + c * C;
         len = std::min(C, sp[k].bytes - c * C);
     };
-    hipError_t err[FETCH_THREADS] = {};
-    // thread k: pieces k, k + T, ...; its two slots in turn
-    auto work = [&](int k) {
-        hipError_t he = hipSetDevice(e->device);
+    // this thread makes the HIP calls; the others empty arrived slots
+    std::atomic<size_t> claimed{0}, arrived{0}, emptied[FETCH_SLOTS];
+    std::atomic<bool> stop{false};
+    for (auto &x : emptied)
+        x = 0;
+    auto empty_slot = [&](size_t c) {
         char *h;
         const char *d;
         size_t len;
-        auto issue = [&](size_t c, int s) {
-            piece(c, h, d, len);
-            if (he == hipSuccess)
-                he = hipMemcpyAsync(e->pin + (2 * k + s) * C, d, len, hipMemcpyDeviceToHost, e->stream);
-            if (he == hipSuccess)
-                he = hipEventRecord(e->pin_ev[2 * k + s], e->stream);
-        };
-        int s = 0;
-        if ((size_t)k < pieces)
-            issue(k, 0);
-        for (size_t c = k; c < pieces && he == hipSuccess; c += T, s ^= 1) {
-            if (c + T < pieces)
-                issue(c + T, s ^ 1);
-            if (he == hipSuccess)
-                he = hipEventSynchronize(e->pin_ev[2 * k + s]);
-            if (he == hipSuccess) {
-                piece(c, h, d, len);
-                std::memcpy(h, e->pin + (2 * k + s) * C, len);
-            }
-        }
-        err[k] = he;
+        piece(c, h, d, len);
+        std::memcpy(h, e->pin + (c % FETCH_SLOTS) * C, len);
+        emptied[c % FETCH_SLOTS].store(c + 1, std::memory_order_release);
     };
-    std::thread th[FETCH_THREADS];
-    bool own[FETCH_THREADS] = {};
-    for (int k = 1; k < T; k++) {
-        try {
-            th[k] = std::thread(work, k);
-        } catch (const std::system_error &) {
-            own[k] = true; // no thread to be had: its pieces are done here
+    auto work = [&]() {
+        for (;;) {
+            const size_t c = claimed.fetch_add(1);
+            if (c >= pieces)
+                return;
+            while (arrived.load(std::memory_order_acquire) <= c) {
+                if (stop.load(std::memory_order_relaxed))
+                    return;
+                __builtin_ia32_pause();
+            }
+            empty_slot(c);
         }
+    };
+    hipError_t he = hipSuccess;
+    size_t issued = 0;
+    auto issue = [&]() {
+        char *h;
+        const char *d;
+        size_t len;
+        piece(issued, h, d, len);
+        const size_t s = issued % FETCH_SLOTS;
+        if (he == hipSuccess)
+            he = hipMemcpyAsync(e->pin + s * C, d, len, hipMemcpyDeviceToHost, e->stream);
+        if (he == hipSuccess)
+            he = hipEventRecord(e->pin_ev[s], e->stream);
+        issued++;
+    };
+    while (issued < pieces && issued < FETCH_SLOTS)
+        issue();
+    meanwhile();
+    std::thread th[FETCH_THREADS];
+    int started = 0;
+    try {
+        for (; started < FETCH_THREADS; started++)
+            th[started] = std::thread(work);
+    } catch (const std::system_error &) {
+        // fewer threads; none: this one empties the slots too
     }
-    work(0);
-    for (int k = 1; k < T; k++) {
-        if (own[k])
-            work(k);
-        else
-            th[k].join();
+    for (size_t c = 0; c < pieces && he == hipSuccess; c++) {
+        // the slots whose pieces have been emptied take the next pieces; piece c
+        // itself is always issued (its slot is waited for)
+        while (issued < pieces && issued < c + FETCH_SLOTS) {
+            std::atomic<size_t> &done = emptied[issued % FETCH_SLOTS];
+            if (done.load(std::memory_order_acquire) != issued - FETCH_SLOTS + 1) {
+                if (issued > c)
+                    break;
+                __builtin_ia32_pause();
+                continue;
+            }
+            issue();
+        }
+        if (he == hipSuccess)
+            he = hipEventSynchronize(e->pin_ev[c % FETCH_SLOTS]);
+        if (he != hipSuccess)
+            break;
+        arrived.store(c + 1, std::memory_order_release);
+        if (!started)
+            empty_slot(c);
     }
+    stop = he != hipSuccess;
+    for (int k = 0; k < started; k++)
+        th[k].join();
+    HIPCHK(he);
     HIPCHK(hipStreamSynchronize(e->stream));
-    for (int k = 0; k < T; k++)
-        HIPCHK(err[k]);
     return MDX_OK;
+}
+
+static int fetch(mdx_engine *e, const Span *sp, int n)
+{
+    return fetch(e, sp, n, false, [] {});
 }
 
 template <class T> static int download(mdx_engine *e, const Buf &b, T *h, size_t n)
@@ -1605,16 +1641,31 @@ static int download_state_t(mdx_engine *e, double *x, double *p, double *Q, doub
     const size_t N = e->N;
     const bool rot = e->integ == MDX_INTEG_ROTOR;
     const int c = e->cur;
-    double *const dst[4] = {x, p, Q, L};
+    double *dst[4] = {x, p, Q, L};
     const int width[4] = {3, 3, 9, 3};
     double *dev[4];
     Span sp[4];
     int n = 0, rc;
+    // beads carry no orientations: identities and zeros, written here, while
+    // the rest is under way, where the threads of the large copies would not
+    // write them faster
+    const bool blank = !rot && 144 * N <= FETCH_SMALL;
+    if (blank)
+        dst[2] = dst[3] = nullptr;
+    auto fill = [&]() {
+        static const double one[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
+        for (size_t i = 0; blank && Q && i < N; i++)
+            std::memcpy(Q + 9 * i, one, sizeof one);
+        if (blank && L)
+            std::memset(L, 0, 24 * N);
+    };
     size_t words = 0;
     for (int k = 0; k < 4; k++)
         words += dst[k] ? width[k] * N : 0;
-    if (words == 0)
+    if (words == 0) {
+        fill();
         return MDX_OK;
+    }
     if ((rc = dalloc(e, e->tmpd, 8 * words)))
         return rc;
     double *at = (double *)e->tmpd.p;
@@ -1630,7 +1681,7 @@ static int download_state_t(mdx_engine *e, double *x, double *p, double *Q, doub
                        rot ? (const R *)e->Q[c].p : nullptr, rot ? (const R *)e->Lm[c].p : nullptr,
                        dev[0], dev[1], dev[2], dev[3]);
     HIPCHK(hipGetLastError());
-    return fetch(e, sp, n, true);
+    return fetch(e, sp, n, true, fill);
 }
 
 int mdx_download_state(mdx_engine *e, double *x, double *p, double *Q, double *L)
