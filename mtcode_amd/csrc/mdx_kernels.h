@@ -656,9 +656,9 @@ __device__ __forceinline__ bool patch_roles(uint32_t oi, int ti, uint32_t oj, in
 // both sides come first, as bit masks, and only the passing patch pairs (one,
 // nearly always) are evaluated: lanes of a wave whose pairs bind through
 // different patches evaluate them together, not one patch pair after the
-// other as a loop over all of them does.
+// other as a loop over all of them does.  Returns how many were evaluated.
 template <class R, int MODE>
-__device__ __forceinline__ void patch_pair(const KArgs<R> &a, const PatchTab &tb, const DevRep &rp,
+__device__ __forceinline__ int patch_pair(const KArgs<R> &a, const PatchTab &tb, const DevRep &rp,
                                            const PosRec &xi, int ti, const R *qi, int j, Acc<R> &acc)
 {
     constexpr bool FP64 = sizeof(R) == 8;
@@ -686,7 +686,7 @@ __device__ __forceinline__ void patch_pair(const KArgs<R> &a, const PatchTab &tb
     const float scr = (float)a.costm_screen_f;
     const uint32_t ma = cone_mask(tb, ta, qs, uf, -1.f, scr);
     if (!ma)
-        return;
+        return 0;
 #pragma unroll
     for (int k = 0; k < 9; k++)
         qs[k] = (float)qc[k];
@@ -695,6 +695,7 @@ __device__ __forceinline__ void patch_pair(const KArgs<R> &a, const PatchTab &tb
     const double *da = tb.dird + 3 * tb.pstart[ta];
     const double *dc = tb.dird + 3 * tb.pstart[tc];
     const int rowbase = rp.prow + tb.rstart[ta * MAXT + tc];
+    int n = 0;
     for (uint32_t m1 = mc ? ma : 0u; m1; m1 &= m1 - 1u) {
         const int ia = __builtin_ctz(m1);
         double n1[3];
@@ -710,6 +711,7 @@ __device__ __forceinline__ void patch_pair(const KArgs<R> &a, const PatchTab &tb
             const double a2 = (n2[0] * u[0] + n2[1] * u[1] + n2[2] * u[2]);
             if (!(a2 > pr.costm))
                 continue;
+            n++;
             R f[3] = {0, 0, 0}, t1[3] = {0, 0, 0}, t2[3] = {0, 0, 0};
             double e;
             if constexpr (FP64) {
@@ -740,6 +742,7 @@ __device__ __forceinline__ void patch_pair(const KArgs<R> &a, const PatchTab &tb
             }
         }
     }
+    return n;
 }
 
 // WCA term of one pair (MD.cpp:1700-1758, potential.h:112-125) into acc:
@@ -1883,6 +1886,328 @@ __global__ void __launch_bounds__(T) k_cstep(KArgs<R> a)
     }
     if (MODE == M_FUSED || MODE == M_BEAD)
         drift_bound(a, drift);
+}
+
+// A force evaluation from the cells (no list) of CG_POS positions in one
+// kernel, for small systems with patches: single-step calls, mdx_prime,
+// mdx_compute_forces and the re-sort steps.  Bound by its chain of dependent
+// loads (start of a row, its slots, their records), not by the chip's width:
+// k_gather's lanes walk their 27 cells and take their patch candidates in
+// turn, 70 us for 512 particles.  Here eight lanes find a position's 9 rows of
+// cells; the candidates of the block's positions are laid out one per lane and
+// those within reach appended in order; then as in k_cstep, one lane per hit
+// and per patch candidate.  One step as a call: 512 tetrahedral particles,
+// mixed, 108 us before, 57 now.  The sums are k_gather's in the same order
+// (the terms of a pair bound through several patch pairs are added one by
+// one), so the results are the same bits.
+constexpr int CG_POS = 16, CG_T = 128, CG_HITS = 512;
+template <class R, int MODE> __global__ void __launch_bounds__(CG_T) k_cgather(KArgs<R> a)
+{
+    constexpr int NPOS = CG_POS, T = CG_T, LP = T / NPOS;
+    static_assert(LP == 8 && T == 128, "8 lanes per position, two waves");
+    static_assert(MODE != M_BEAD, "systems with patches");
+    __shared__ PosRec sx[NPOS];
+    __shared__ float sq[NPOS * 9];
+    __shared__ int sslot[NPOS], sexc[NPOS * 2];
+    __shared__ unsigned char sbad[NPOS];
+    // list ranges of a position's rows (two per row) and their candidates'
+    // first numbers; first candidate of each position
+    __shared__ int rbeg[NPOS][18], rcum[NPOS][18], off[NPOS + 1];
+    __shared__ int hslot[CG_HITS];
+    __shared__ unsigned char hown[CG_HITS];
+    __shared__ int hbeg[NPOS], hend[NPOS];
+    __shared__ unsigned char own[CS_CAND * NPOS];
+    __shared__ int poff[NPOS];
+    __shared__ R ent[T * 6];
+    __shared__ int pj[T];
+    __shared__ int plist[CS_CAND * NPOS];
+    __shared__ int wcount[2], stotal;
+    __shared__ PatchTab tb;
+    load_tab(a, tb);
+    const int tid = threadIdx.x;
+    const int base = xcd_block(blockIdx.x, gridDim.x) * NPOS;
+    {
+        const int pos = tid / LP, sub = tid % LP;
+        const bool livep = base + pos < a.N;
+        int len0 = 0, len1 = 0, b0 = 0, b1 = 0, l80 = 0, l81 = 0, b80 = 0, b81 = 0;
+        if (livep) {
+            const int i = a.list[base + pos];
+            const PosRec xi = a.X[i];
+            const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xi.meta >> 8];
+            const int n0 = rp.nc[0], n1 = rp.nc[1], n2 = rp.nc[2];
+            const int c = a.cell[i] - rp.coff;
+            const int cx = c % n0, cy = (c / n0) % n1, cz = c / (n0 * n1);
+            // row k: z offset k / 3 - 1, y offset k % 3 - 1 (the stencil and the
+            // order of for_each_in_cells)
+            auto row = [&](int k, int &r0, int &m0, int &r2, int &m2) {
+                const int oz = k / 3 - 1, oy = k % 3 - 1;
+                r0 = m0 = r2 = m2 = 0;
+                if ((oz < 0 && n2 < 3) || (oz > 0 && n2 < 2) || (oy < 0 && n1 < 3) ||
+                    (oy > 0 && n1 < 2))
+                    return;
+                int z = cz + oz, y = cy + oy;
+                z = z < 0 ? z + n2 : (z >= n2 ? z - n2 : z);
+                y = y < 0 ? y + n1 : (y >= n1 ? y - n1 : y);
+                const int *st = a.start + rp.coff + n0 * (y + n1 * z);
+                if (n0 < 3) {
+                    r0 = st[0];
+                    m0 = st[n0] - r0;
+                } else if (cx == 0) {
+                    r0 = st[0];
+                    m0 = st[2] - r0;
+                    r2 = st[n0 - 1];
+                    m2 = st[n0] - r2;
+                } else if (cx == n0 - 1) {
+                    r0 = st[n0 - 2];
+                    m0 = st[n0] - r0;
+                    r2 = st[0];
+                    m2 = st[1] - r2;
+                } else {
+                    r0 = st[cx - 1];
+                    m0 = st[cx + 2] - r0;
+                }
+            };
+            row(sub, b0, len0, b1, len1);
+            if (sub == 0) {
+                row(8, b80, l80, b81, l81);
+                sx[pos] = xi;
+                sslot[pos] = i;
+                sbad[pos] = 0;
+                const bool ne = needs_exclusions(a, i);
+                sexc[2 * pos] = ne ? a.exc_off[xi.id] : 0;
+                sexc[2 * pos + 1] = ne ? a.exc_off[xi.id + 1] : 0;
+                R qm[9];
+                load_orient(a.Q, (size_t)i, qm);
+#pragma unroll
+                for (int k = 0; k < 9; k++)
+                    sq[9 * pos + k] = (float)qm[k];
+            }
+        }
+        // candidates before each row: a prefix over the position's lanes
+        int v = len0 + len1;
+        for (int o = 1; o < LP; o <<= 1) {
+            const int u = __shfl_up(v, o, LP);
+            if (sub >= o)
+                v += u;
+        }
+        const int eight = __shfl(v, LP - 1, LP);
+        const int first = v - len0 - len1;
+        rbeg[pos][2 * sub] = b0;
+        rcum[pos][2 * sub] = first;
+        rbeg[pos][2 * sub + 1] = b1;
+        rcum[pos][2 * sub + 1] = first + len0;
+        if (sub == 0) {
+            rbeg[pos][16] = b80;
+            rcum[pos][16] = eight;
+            rbeg[pos][17] = b81;
+            rcum[pos][17] = eight + l80;
+            off[pos + 1] = eight + l80 + l81;
+        }
+    }
+    __syncthreads();
+    if (tid < 64) {
+        int v = tid < NPOS ? off[tid + 1] : 0;
+        for (int o = 1; o < NPOS; o <<= 1) {
+            const int u = __shfl_up(v, o);
+            if (tid >= o)
+                v += u;
+        }
+        if (tid < NPOS)
+            off[tid + 1] = v; // (one wave: every lane has read its count)
+        if (tid == 0)
+            off[0] = 0;
+    }
+    __syncthreads();
+    const int total = off[NPOS];
+    const int s = base + tid;
+    const bool live = tid < NPOS && s < a.N;
+    R F[3] = {0, 0, 0}, Tq[3] = {0, 0, 0};
+    int c0 = 0, more = 0; // patch candidates of a position taken by earlier passes
+    do {
+        int npc = 0, nhit = 0;
+        for (int r0 = 0; r0 < total || (r0 == 0 && total == 0); r0 += T) {
+            // this round's candidates within reach, appended in order
+            const int e = r0 + tid;
+            bool hit = false;
+            int o = 0, j = 0;
+            if (e < total) {
+                int lo = 0, hi = NPOS - 1;
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (off[mid] <= e)
+                        lo = mid;
+                    else
+                        hi = mid - 1;
+                }
+                o = lo;
+                const int f = e - off[o];
+                lo = 0;
+                hi = 17;
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (rcum[o][mid] <= f)
+                        lo = mid;
+                    else
+                        hi = mid - 1;
+                }
+                j = a.list[rbeg[o][lo] + f - rcum[o][lo]];
+                if (j != sslot[o]) {
+                    const PosRec xj = a.X[j];
+                    const PosRec xo = sx[o];
+                    const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xo.meta >> 8];
+                    double d[3];
+                    min_image(a, rp, xo.x, xo.y, xo.z, xj, d);
+                    hit = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] < a.rmax2;
+                }
+            }
+            const unsigned long long m = __ballot(hit);
+            if ((tid & 63) == 0)
+                wcount[tid >> 6] = __popcll(m);
+            __syncthreads();
+            if (hit) {
+                const int at = nhit + (tid >= 64 ? wcount[0] : 0) +
+                               __popcll(m & ((1ull << (tid & 63)) - 1ull));
+                hslot[at] = j;
+                hown[at] = (unsigned char)o;
+            }
+            nhit += wcount[0] + wcount[1];
+            if (tid < NPOS)
+                hbeg[tid] = hend[tid] = 0;
+            __syncthreads();
+            if (r0 + T < total && nhit <= CG_HITS - T)
+                continue;
+            // the hits so far: where each position's begin and end, then one per
+            // lane
+            for (int h = tid; h < nhit; h += T) {
+                if (h == 0 || hown[h] != hown[h - 1])
+                    hbeg[hown[h]] = h;
+                if (h == nhit - 1 || hown[h] != hown[h + 1])
+                    hend[hown[h]] = h + 1;
+            }
+            for (int h0 = 0; h0 < nhit; h0 += T) {
+                const int h = h0 + tid;
+                if (h < nhit) {
+                    const int ho = hown[h], hj = hslot[h];
+                    const PosRec xj = a.X[hj];
+                    const PosRec xo = sx[ho];
+                    const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xo.meta >> 8];
+                    double d[3];
+                    min_image(a, rp, xo.x, xo.y, xo.z, xj, d);
+                    const double r2s = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+                    Acc<R> pa;
+                    pa.F[0] = pa.F[1] = pa.F[2] = 0;
+                    pa.bad = false;
+                    wca_term<R, MODE>(a, d, r2s, xj.id, sexc[2 * ho], sexc[2 * ho + 1], pa);
+                    bool c = false;
+                    if (r2s < a.maxd2) {
+                        const int to = xo.meta & 255, tj = xj.meta & 255;
+                        int ta, tc;
+                        patch_roles(xo.id, to, xj.id, tj, ta, tc);
+                        c = tb.np[to] > 0 && tb.np[tj] > 0 &&
+                            ((a.active_mask >> (ta * MAXT + tc)) & 1ull) &&
+                            own_screen(a, tb, to, sq + 9 * ho, d, r2s);
+                    }
+                    for (int k = 0; k < 3; k++)
+                        ent[3 * tid + k] = pa.F[k];
+                    if (pa.bad)
+                        sbad[ho] = 1;
+                    pj[tid] = c ? hj : -1;
+                }
+                __syncthreads();
+                if (tid < NPOS)
+                    for (int h2 = max(hbeg[tid], h0); h2 < min(hend[tid], h0 + T); h2++) {
+                        if (c0 == 0)
+                            for (int k = 0; k < 3; k++)
+                                F[k] += ent[3 * (h2 - h0) + k];
+                        const int jc = pj[h2 - h0];
+                        if (jc >= 0) {
+                            if (npc >= c0 && npc < c0 + CS_CAND)
+                                plist[(npc - c0) * NPOS + tid] = jc;
+                            npc++;
+                        }
+                    }
+                __syncthreads();
+            }
+            nhit = 0;
+        }
+        // this pass's patch candidates, one per lane
+        const int nq = tid < NPOS ? max(0, min(npc - c0, CS_CAND)) : 0;
+        int first = nq;
+        if (tid < 64) {
+            for (int o = 1; o < NPOS; o <<= 1) {
+                const int u = __shfl_up(first, o);
+                if (tid >= o)
+                    first += u;
+            }
+            if (tid == NPOS - 1)
+                stotal = first;
+            first -= nq;
+        }
+        if (tid < NPOS) {
+            poff[tid] = first;
+            for (int k = 0; k < nq; k++)
+                own[first + k] = (unsigned char)tid;
+        }
+        __syncthreads();
+        const int ncand = stotal; // (at most CS_CAND * NPOS = T: one round)
+        static_assert(CS_CAND * CG_POS <= CG_T, "the candidates of a pass fit one round");
+        if (tid < ncand) {
+            const int o = own[tid], i = sslot[o];
+            const PosRec xo = sx[o];
+            const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xo.meta >> 8];
+            R qo[9];
+            load_orient(a.Q, (size_t)i, qo);
+            Acc<R> ea;
+            for (int k = 0; k < 3; k++)
+                ea.F[k] = ea.T[k] = 0;
+            ea.bad = false;
+            const int j = plist[(tid - poff[o]) * NPOS + o];
+            const int n = patch_pair<R, MODE>(a, tb, rp, xo, xo.meta & 255, qo, j, ea);
+            pj[tid] = n > 1 ? j : -1;
+            for (int k = 0; k < 3; k++) {
+                ent[6 * tid + k] = ea.F[k];
+                ent[6 * tid + 3 + k] = ea.T[k];
+            }
+        }
+        __syncthreads();
+        for (int q = 0; q < nq; q++) {
+            const int j = pj[first + q];
+            if (j >= 0) {
+                // several patch pairs bind: their terms one by one, as the
+                // one-lane kernel adds them
+                const PosRec xo = sx[tid];
+                const DevRep &rp = a.nrep == 1 ? a.reps[0] : a.reps[xo.meta >> 8];
+                R qo[9];
+                load_orient(a.Q, (size_t)sslot[tid], qo);
+                Acc<R> sa;
+                for (int k = 0; k < 3; k++) {
+                    sa.F[k] = F[k];
+                    sa.T[k] = Tq[k];
+                }
+                sa.bad = false;
+                patch_pair<R, MODE>(a, tb, rp, xo, xo.meta & 255, qo, j, sa);
+                for (int k = 0; k < 3; k++) {
+                    F[k] = sa.F[k];
+                    Tq[k] = sa.T[k];
+                }
+                continue;
+            }
+            for (int k = 0; k < 3; k++) {
+                F[k] += ent[6 * (first + q) + k];
+                Tq[k] += ent[6 * (first + q) + 3 + k];
+            }
+        }
+        c0 += CS_CAND;
+        more = __syncthreads_or(tid < NPOS && npc > c0);
+    } while (more);
+    float drift = 0.f;
+    if (live) {
+        const R fin[6] = {F[0], F[1], F[2], Tq[0], Tq[1], Tq[2]};
+        process_particle<R, MODE, PH_INTEGRATE_F>(
+            a, nullptr, s, nullptr,
+            [&](int i, const DevRep &rp, auto &&fn) { for_each_near(a, rp, i, fn); }, drift, fin,
+            sbad[tid] != 0);
+    }
 }
 
 // ... then the patch pairs, topology and the integrator
