@@ -2298,14 +2298,22 @@ __global__ void __launch_bounds__(256) k_patch(KArgs<R> a, int pblk)
     load_tab(a, tb);
     const int tid = threadIdx.x;
     const int base = xcd_block(blockIdx.x, gridDim.x) * pblk;
-    // exclusive scan of min(ncand, pcap) in position order (position
-    // k * 256 + tid of the block, k < PER)
-    int carry = 0;
-    for (int k = 0; k < PER; k++) {
-        const int p = base + k * 256 + tid;
-        const int nc = p < a.N ? a.ncand[p] : 0;
-        const int nq = nc < a.pcap ? nc : a.pcap;
-        int v = nq;
+    // exclusive scan of min(ncand, pcap) in position order: a thread takes PER
+    // consecutive positions, their counts loaded together, then one scan over
+    // the block (a scan per 256 positions, each after its own load, was 6 of
+    // the 16.1 us at 1,048,576 particles with 2,048 positions per block; 12.9
+    // now, and 11.9 -> 11.2 for 64 replicas of 512 to 16,384)
+    int carry;
+    {
+        int nq[PBLK / 256], mine = 0;
+#pragma unroll
+        for (int k = 0; k < PBLK / 256; k++) {
+            const int p = base + tid * PER + k;
+            const int nc = k < PER && p < a.N ? a.ncand[p] : 0;
+            nq[k] = nc < a.pcap ? nc : a.pcap;
+            mine += nq[k];
+        }
+        int v = mine;
         for (int o = 1; o < 64; o <<= 1) {
             const int t = __shfl_up(v, o);
             if ((tid & 63) >= o)
@@ -2314,12 +2322,16 @@ __global__ void __launch_bounds__(256) k_patch(KArgs<R> a, int pblk)
         if ((tid & 63) == 63)
             wsum[tid >> 6] = v;
         __syncthreads();
-        int wb = 0;
+        int at = v - mine;
         for (int w = 0; w < (tid >> 6); w++)
-            wb += wsum[w];
-        off[k * 256 + tid] = carry + wb + v - nq;
-        carry += wsum[0] + wsum[1] + wsum[2] + wsum[3];
-        __syncthreads();
+            at += wsum[w];
+#pragma unroll
+        for (int k = 0; k < PBLK / 256; k++)
+            if (k < PER) {
+                off[tid * PER + k] = at;
+                at += nq[k];
+            }
+        carry = wsum[0] + wsum[1] + wsum[2] + wsum[3];
     }
     if (tid == 0)
         off[pblk] = carry;
