@@ -361,12 +361,12 @@ def main():
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": traffic,
             "kernel": ("one step: k_walkc (WCA) + k_bind_edges + k_bind_decide + k_bind_forces "
-                       "+ k_integrate + list upkeep (gated; amortised) + k_decide"
+                       "+ k_integrate + list upkeep (k_upkeep, k_nbuild, gated; amortised)"
                        if s.get("binding") else
-                       "one step: k_walkc + k_patch + k_integrate + list upkeep (k_bin, k_scan1, "
-                       "k_scan3, k_fill, k_cellsort, k_nbuild, gated; amortised) + k_decide"
+                       "one step: k_walkc + k_patch + k_integrate + list upkeep (k_upkeep, "
+                       "k_nbuild, gated; amortised)"
                        if "walk" in prof else
-                       "one step: k_gather + list upkeep (gated; amortised) + k_decide"),
+                       "one step: k_cstep + list upkeep (k_upkeep, k_nbuild, gated; amortised)"),
             "algorithmic_bytes_per_particle_step": algo["mixed"],
             "step_kernel_ms": step_ms,
             "per_kernel": per_kernel,
