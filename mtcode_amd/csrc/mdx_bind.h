@@ -49,15 +49,15 @@ struct BindArgs {
     int *adj_n;       // candidates per patch
     int *adj_p;       // partner patches, BIND_DEG per patch, ascending
     double *adj_s;    // their scores
-    int nh;
     double mk2;       // squared largest interaction distance (max_check)
     double cmin;      // smallest cos(theta_m) of any row (the cone screen)
     double on_rate, off_rate;
     uint32_t key0, key1;
     unsigned long long draw;
+    StepCtl *ctl;
+    int nh;         // patches
     int draw_epoch; // 1: the draw counter is the force-evaluation count (steps)
     int ep_off;     // 1: that count already includes this evaluation (list steps)
-    StepCtl *ctl;
     // 0: BindingModelSingle(on_rate, off_rate); 1: the species-table form of
     // BindingModelBinary / BindingModelTernary: species[patch] in 1..3,
     // dtab[pair * 4 + 2 * before + k] (k 0: rate to unbound, 1: to bound) by
@@ -68,6 +68,8 @@ struct BindArgs {
     const int *species;
     const double *dtab, *ttab, *tr4;
 };
+// (compared byte by byte in the key of the captured steps)
+static_assert(sizeof(BindArgs) == 20 * 8, "no padding");
 
 // status bit 3: a patch with more than BIND_DEG candidates, or a component
 // of more than BIND_CMAX patches

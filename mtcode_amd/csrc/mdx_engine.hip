@@ -757,6 +757,7 @@ template <class R> static int bin_current(mdx_engine *e)
 
 template <class R, int MODE>
 static int launch_bind_step(mdx_engine *e, const double *noise_dev, int lmode);
+template <class R> static BindArgs bind_args(mdx_engine *e, unsigned long long draw);
 
 template <class R> static void topo_args(const mdx_engine *e, KArgs<R> &a);
 
@@ -1172,15 +1173,25 @@ template <class R, int MODE> static int list_step_graph(mdx_engine *e, int steps
     KArgs<R> a = make_args<R>(e);
     a.lmode = 1;
     topo_args(e, a);
-    // the arguments, the grid and the launch-form switches (which kernels
-    // the step launches)
-    const int form[7] = {e->ncells,      e->N,         e->use_split, e->use_compact,
-                         e->use_walkc,   e->use_fuse,  e->use_tiles};
-    const double rates[3] = {e->bind_on_rate, e->bind_off_rate, (double)e->bind_table};
-    std::vector<char> sig(sizeof a + sizeof form + sizeof rates);
-    memcpy(sig.data(), &a, sizeof a);
-    memcpy(sig.data() + sizeof a, form, sizeof form);
-    memcpy(sig.data() + sizeof a + sizeof form, rates, sizeof rates);
+    // the arguments, the grid, what decides which kernels the step launches
+    // (n_patchy: the fused form), and under binding the arguments of its
+    // kernels, whose grids and arrays follow the patch numbering
+    const int form[8] = {e->ncells,    e->N,        e->use_split, e->use_compact,
+                         e->use_walkc, e->use_fuse, e->use_tiles, e->n_patchy};
+    BindArgs b;
+    memset(&b, 0, sizeof b);
+    const void *bft[2] = {nullptr, nullptr};
+    if (e->bind_on) {
+        b = bind_args<R>(e, 0);
+        bft[0] = e->bF.p;
+        bft[1] = e->bT.p;
+    }
+    std::vector<char> sig(sizeof a + sizeof form + sizeof b + sizeof bft);
+    char *at = sig.data();
+    memcpy(at, &a, sizeof a);
+    memcpy(at += sizeof a, form, sizeof form);
+    memcpy(at += sizeof form, &b, sizeof b);
+    memcpy(at + sizeof b, bft, sizeof bft);
     GraphSlot &g = e->graphs[steps > 1][e->cur];
     if (!g.exec || g.sig != sig) {
         if (g.exec) {
