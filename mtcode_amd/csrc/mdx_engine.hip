@@ -1790,7 +1790,7 @@ static int patch_rows_upload(mdx_engine *e)
                 e->active_mask |= 1ull << (ta * MAXT + tc);
         }
     e->grid_dirty = true;
-    return upload(e, e->prows, rows.data(), std::max<size_t>(rows.size(), 1));
+    return upload(e, e->prows, rows.data(), rows.size());
 }
 
 int mdx_set_patches(mdx_engine *e, int ntypes, const int *type_of_particle,
@@ -2048,7 +2048,7 @@ int mdx_set_exclusions(mdx_engine *e, long long npairs, const int *ij)
             return set_err(MDX_ERR_ARG, "particle %d has more than %d exclusions", i, MAXEXCL);
     int rc;
     if ((rc = upload(e, e->exc_off, off.data(), off.size())) ||
-        (rc = upload(e, e->exc_j, val.data(), std::max<size_t>(val.size(), 1))))
+        (rc = upload(e, e->exc_j, val.data(), val.size())))
         return rc;
     e->nexcl = npairs;
     return MDX_OK;
