@@ -2051,6 +2051,9 @@ int mdx_set_exclusions(mdx_engine *e, long long npairs, const int *ij)
         (rc = upload(e, e->exc_j, val.data(), val.size())))
         return rc;
     e->nexcl = npairs;
+    // a list holds no pair that was excluded when it was built, and its walk
+    // does not look for exclusions where it holds none
+    e->list_valid = false;
     return MDX_OK;
 }
 
