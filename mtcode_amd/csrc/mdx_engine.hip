@@ -2141,9 +2141,9 @@ int mdx_cell_assign(mdx_engine *e, int replica, const int n[3], int *cell_of)
 
 // positions of replica r in original order (tmpx), their cells on an
 // n[0] x n[1] x n[2] grid (tmpi), that grid's cell list (tmpi3: starts, tmpi2:
-// members, in original order if ordered) and the positions in the list's order
-// (asorted, written before the ordering); a parity / analysis path, not the step
-static int custom_cells(mdx_engine *e, int replica, const int n[3], bool ordered)
+// members in order of arrival) and the positions in the list's order (asorted);
+// a parity / analysis path, not the step
+static int custom_cells(mdx_engine *e, int replica, const int n[3])
 {
     const long long nc = (long long)n[0] * n[1] * n[2];
     if (nc > (1ll << 28))
@@ -2154,8 +2154,8 @@ static int custom_cells(mdx_engine *e, int replica, const int n[3], bool ordered
     if ((rc = replica_positions(e, replica)) || (rc = dalloc(e, e->tmpi, 4 * (size_t)cnt)) ||
         (rc = dalloc(e, e->tmpi2, 4 * (size_t)cnt)) || (rc = dalloc(e, e->tmpi3, 4 * (size_t)(nc + 1))))
         return rc;
-    // counted, scanned, filled and ordered on the device (through the host the
-    // lists of two grids took 0.8 ms for 100,003 particles)
+    // counted, scanned and filled on the device (through the host the lists of
+    // two grids took 0.8 ms for 100,003 particles)
     const int ncell = (int)nc, nb = (ncell + 1023) / 1024;
     if ((rc = dalloc(e, e->arank, 4 * (size_t)cnt)) || (rc = dalloc(e, e->acount, 4 * (size_t)ncell)) ||
         (rc = dalloc(e, e->absum, 4 * (size_t)nb)) ||
@@ -2173,10 +2173,6 @@ static int custom_cells(mdx_engine *e, int replica, const int n[3], bool ordered
     hipLaunchKernelGGL(k_fill_custom, dim3(nblk(cnt)), dim3(256), 0, e->stream,
                        (const double *)e->tmpx.p, cnt, (const int *)cell, (const int *)e->arank.p,
                        (const int *)start, list, (PosRec *)e->asorted.p);
-    if (ordered)
-        hipLaunchKernelGGL(k_cellsort, dim3(nblk(cnt)), dim3(256), 0, e->stream, cnt,
-                           (const int *)cell, (const int *)e->arank.p, (const int *)start, list,
-                           (const PosRec *)nullptr);
     HIPCHK(hipGetLastError());
     return MDX_OK;
 }
@@ -2214,7 +2210,7 @@ int mdx_pair_histogram(mdx_engine *e, int replica, double max, double dx, long l
             d2 = std::nextafter(d2, HUGE_VAL);
         edge[(size_t)k] = d2;
     }
-    if ((rc = custom_cells(e, replica, n, false)) ||
+    if ((rc = custom_cells(e, replica, n)) ||
         (rc = dalloc(e, e->tmpll, 8 * (size_t)std::max(gs, 1))) ||
         (rc = upload(e, e->aedge, edge.data(), edge.size())))
         return rc;
@@ -2269,13 +2265,19 @@ static int pair_list(mdx_engine *e, int replica, const int n[3], double cut, Buf
     const int cnt = e->nper[replica];
     const double *b = &e->box[3 * replica];
     int rc;
-    if ((rc = custom_cells(e, replica, n, true)) || (rc = dalloc(e, e->tmpll, 8 * (size_t)(cnt + 1))) ||
+    if ((rc = custom_cells(e, replica, n)) || (rc = dalloc(e, e->tmpll, 8 * (size_t)(cnt + 1))) ||
         (rc = dalloc(e, e->partial, 4 * (size_t)cnt)))
         return rc;
     const double *X = (const double *)e->tmpx.p;
+    // the members of each cell in ascending order (k_pairs then finds most
+    // partners in order), into the ranks' array
+    int *list = (int *)e->arank.p;
+    hipLaunchKernelGGL(k_order_custom, dim3(nblk(cnt)), dim3(256), 0, e->stream, cnt,
+                       (const int *)e->tmpi.p, (const int *)e->tmpi3.p, (const int *)e->tmpi2.p,
+                       list);
     hipLaunchKernelGGL(k_pairs, dim3(nblk(cnt)), dim3(256), 0, e->stream, X, cnt, b[0], b[1],
                        b[2], e->periodic, n[0], n[1], n[2], cut, (const int *)e->tmpi.p,
-                       (const int *)e->tmpi3.p, (const int *)e->tmpi2.p, (int *)e->partial.p,
+                       (const int *)e->tmpi3.p, (const int *)list, (int *)e->partial.p,
                        (const long long *)nullptr, (int *)nullptr, 0ll, 0);
     HIPCHK(hipGetLastError());
     std::vector<int> pc(cnt);
@@ -2292,7 +2294,7 @@ static int pair_list(mdx_engine *e, int replica, const int n[3], double cut, Buf
             return rc;
         hipLaunchKernelGGL(k_pairs, dim3(nblk(cnt)), dim3(256), 0, e->stream, X, cnt, b[0],
                            b[1], b[2], e->periodic, n[0], n[1], n[2], cut, (const int *)e->tmpi.p,
-                           (const int *)e->tmpi3.p, (const int *)e->tmpi2.p, (int *)nullptr,
+                           (const int *)e->tmpi3.p, (const int *)list, (int *)nullptr,
                            (const long long *)e->tmpll.p, (int *)out.p, w, 1);
         HIPCHK(hipGetLastError());
     }
@@ -2342,7 +2344,7 @@ int mdx_clusters(mdx_engine *e, int replica, const int n[3], double cut, int ex_
     const int cnt = e->nper[replica];
     const double *b = &e->box[3 * replica];
     int rc;
-    if ((rc = custom_cells(e, replica, n, false)) || (rc = dalloc(e, e->alab, 4 * (size_t)cnt)))
+    if ((rc = custom_cells(e, replica, n)) || (rc = dalloc(e, e->alab, 4 * (size_t)cnt)))
         return rc;
     int *lab = (int *)e->alab.p;
     hipLaunchKernelGGL(k_cc_init, dim3(nblk(cnt)), dim3(256), 0, e->stream, lab, cnt);

@@ -3223,7 +3223,6 @@ __global__ void __launch_bounds__(256) k_fill(int N, const int *cell, const int 
 // the floating-point sums, independent of atomic arrival order and of the
 // slot numbering (a state uploaded in original order and the same state held
 // in cell order walk their cells, and build their lists, in the same order).
-// Without X the members are sorted by their own value.
 // The particle that arrived first in its cell (rank 0, unique per non-empty
 // cell and not changed by the sort) sorts the cell, so empty cells cost
 // nothing.
@@ -3236,9 +3235,9 @@ __device__ __forceinline__ void cellsort_one(const int *cell, const int *rank, c
     const int s0 = start[c], s1 = start[c + 1];
     for (int s = s0 + 1; s < s1; s++) {
         const int v = list[s];
-        const uint32_t idv = X ? X[v].id : (uint32_t)v;
+        const uint32_t idv = X[v].id;
         int t = s - 1;
-        while (t >= s0 && (X ? X[list[t]].id : (uint32_t)list[t]) > idv) {
+        while (t >= s0 && X[list[t]].id > idv) {
             list[t + 1] = list[t];
             t--;
         }
@@ -3614,6 +3613,26 @@ __global__ void __launch_bounds__(256) k_fill_custom(const double *X, int count,
     r.meta = (uint32_t)cell[k];
     list[at] = k;
     sorted[at] = r;
+}
+
+// the members of each cell in ascending order: a particle's place is the number
+// of smaller members, counted by its own thread (the lanes of a wave mostly read
+// the same cell).  A grid may hold any number of particles per cell, and one
+// lane that sorts a cell takes the square of that number in dependent loads
+// (1,000 particles in one cell: 40 ms).  This reads a particle's own cell once;
+// the search that follows reads the neighbouring ones twice.
+__global__ void __launch_bounds__(256) k_order_custom(int count, const int *cell, const int *start,
+                                                      const int *list, int *ordered)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= count)
+        return;
+    const int s0 = start[cell[k]], s1 = start[cell[k] + 1];
+    int at = s0;
+#pragma unroll 8
+    for (int s = s0; s < s1; s++)
+        at += list[s] < k ? 1 : 0;
+    ordered[at] = k;
 }
 
 // fn(record) for every particle after position q of the cell order in the
