@@ -1093,9 +1093,7 @@ template <class R> static int upkeep(mdx_engine *e)
 }
 
 // neighbour list of the current slots from the cell list just built
-// (exact: only pairs within the list radii in FP64)
-template <class R>
-static int build_list(mdx_engine *e, const int *cells, int gated, bool exact = false)
+template <class R> static int build_list(mdx_engine *e, const int *cells, int gated)
 {
     KArgs<R> a = make_args<R>(e);
     a.lmode = 1;
@@ -1112,16 +1110,18 @@ static int build_list(mdx_engine *e, const int *cells, int gated, bool exact = f
         e->nb_dense >= 0
             ? e->nb_dense != 0
             : per_row > 0 && (std::ceil(256.0 / per_row) + 3.0) * per_row > 0.9 * NB_CAP_S;
-    // error of an FP32 squared distance near the list radius rl: coordinates
-    // and box edges are off by up to 2^-24 L each, so a component by 3 of
-    // these, the square by 2 sqrt(3) rl times that, and 4 roundings of rl^2:
-    // below 11 * 2^-24 (L + rl) rl.  Nearly three times that is added
-    const double rl = std::sqrt(a.rl2), slack = 32 * 5.97e-8 * (lmax + rl) * rl;
-    const float rl2f = (float)(a.rl2 + slack), rl2wf = (float)(a.rl2w + slack);
+    // FP32 distances of coordinates within twice the box edge L, against a list
+    // radius rl: a component is off by at most 6 * 2^-24 (L + rl) (two
+    // coordinates by 2 each, the edge and the difference by 1), less than E, so
+    // a distance by less than sqrt(3) E; E also covers the roundings of the square
+    const double rl = std::sqrt(a.rl2), E = 8 * 5.97e-8 * (lmax + rl);
+    const double slack = 2 * std::sqrt(3.0) * rl * E + 3 * E * E;
+    const NbBand bd = {(float)(a.rl2 - slack), (float)(a.rl2 + slack), (float)(a.rl2w - slack),
+                       (float)(a.rl2w + slack)};
     const dim3 blk(256);
 #define NBUILD(CAP, LP)                                                                          \
     hipLaunchKernelGGL((k_nbuild<R, CAP, LP>), dim3(nblk(e->N, 256 / LP)), blk, 0, e->stream, a,  \
-                       cells, gated, exact ? 1 : 0, rl2f, rl2wf)
+                       cells, gated, bd)
     // four lanes per position while the longest lane bounds the build (us per
     // step with 4 / 1 lanes, tetrahedral and condensate, mixed: 4,000 particles
     // 21.7 / 24.0 and 20.5 / 23.1, 70,000 47.9 / 50.1 and 36.5 / 38.0, 130,000
@@ -3045,7 +3045,7 @@ static int list_pairs_t(mdx_engine *e, int *ij, long long cap, long long *npairs
         return rc;
     if (!e->counted && (rc = count_current<R>(e)))
         return rc;
-    if ((rc = finish_bins(e)) || (rc = build_list<R>(e, (const int *)e->cell[e->cur].p, 0, true)))
+    if ((rc = finish_bins(e)) || (rc = build_list<R>(e, (const int *)e->cell[e->cur].p, 0)))
         return rc;
     e->counted = false;
     e->binned = true;

@@ -2486,10 +2486,9 @@ __global__ void __launch_bounds__(256) k_integrate(KArgs<R> a)
 // -- are one contiguous run.  The walk first marks the candidates within the
 // list radius in a bit mask (a distance per candidate, no other work), then
 // takes the marked ones in order.  The marks are FP32 distances against the
-// radius plus a bound on their error (rl2f, rl2wf: the host's), so a list holds
-// every pair within the radius and may hold a few just beyond it, which add
-// nothing to any sum (the walk's own FP64 cut-offs are shorter by the skin);
-// exact: those are left out again by their FP64 distance (mdx_list_pairs).
+// radius plus a bound on their error; a marked pair whose FP32 distance lies
+// within that bound of a radius is decided by its FP64 distance (NbBand), so the
+// list is the set of pairs within the radii in FP64 (mdx_list_pairs).
 // With FP64 records staged (32 B, two LDS reads per candidate, 38 KB) the walk
 // was bound by LDS reads and by 4 blocks per CU.  A block whose particles span more than NB_W rows or two
 // replicas, a grid with fewer than 3 cells on a side, and a z offset whose
@@ -2535,13 +2534,20 @@ __device__ __forceinline__ void row_ranges(const T *off, int n0, int cx, int &r0
     }
 }
 
+// Squared FP32 distances of k_nbuild: from hi on beyond the list radius, below
+// lo within it; below wlo within the radius of the type pairs without patch
+// terms, from whi on beyond that.  Between, the FP64 distance decides.
+struct NbBand {
+    float lo, hi, wlo, whi;
+};
+
 // The sparse one-lane form is held to 80 VGPRs (6 waves per SIMD, no spill: 120
 // -> 106 us).  Measured, a rebuild's list: 1,048,576-particle condensate 145
 // (FP64 records) -> 106 us, 64 replicas (298,897) 98 -> 76, 262,144 polymer
 // beads 68 -> 61, 4,096 particles 42 -> 19 (four lanes per position).
 template <class R, int NB_CAP, int LP>
-__global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1) k_nbuild(KArgs<R> a, const int *cells, int gated, int exact,
-                                                float rl2f, float rl2wf)
+__global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1)
+    k_nbuild(KArgs<R> a, const int *cells, int gated, NbBand bd)
 {
     if (gated && !a.ctl->rebuild)
         return;
@@ -2706,12 +2712,18 @@ __global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1) k_
         const int cy = (cc / n0) % n1, cz = cc / (n0 * n1);
         plain = !a.periodic || (n0 >= 5 && n1 >= 5 && n2 >= 5 && cx >= 1 && cx <= n0 - 2 &&
                                 cy >= 1 && cy <= n1 - 2 && cz >= 1 && cz <= n2 - 2);
-        const float xf[3] = {(float)xi.x, (float)xi.y, (float)xi.z};
         float lf[3], hf[3]; // box edges and their halves (walls: never reached)
         for (int k = 0; k < 3; k++) {
             lf[k] = (float)rb.l[k];
             hf[k] = a.periodic ? 0.5f * lf[k] : 3.0e38f;
         }
+        // (NaN beyond twice the edge, where the bands do not hold: the FP64
+        // distance decides every candidate of such a particle)
+        auto coarse = [&](double x, int k) -> float {
+            const float v = (float)x;
+            return fabsf(v) <= 2.f * lf[k] ? v : __uint_as_float(0x7fc00000u);
+        };
+        const float xf[3] = {coarse(xi.x, 0), coarse(xi.y, 1), coarse(xi.z, 2)};
         const int wv = tid >> 6, lane = tid & 63;
         // wave p (z offset p - 1): the candidate rows, own row rf + m / 3
         // moved by m % 3 - 1 in y and by p - 1 in z; the distinct ones are
@@ -2811,7 +2823,7 @@ __global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1) k_
                     const PosRec xj = a.X[j];
                     lslot[f] = j;
                     ltype[f] = (unsigned char)xj.meta;
-                    lpos[f] = make_float4((float)xj.x, (float)xj.y, (float)xj.z,
+                    lpos[f] = make_float4(coarse(xj.x, 0), coarse(xj.y, 1), coarse(xj.z, 2),
                                           __uint_as_float(xj.id));
                 }
             __syncthreads();
@@ -2851,9 +2863,9 @@ __global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1) k_
                     for (int t = t0 + sub; t < te; t += 2 * LP) {
                         const bool two = t + LP < te;
                         const float4 v0 = lpos[at(t)], v1 = lpos[at(two ? t + LP : t)];
-                        if (dist2f(v0) < rl2f && __float_as_uint(v0.w) != xi.id)
+                        if (!(dist2f(v0) >= bd.hi) && __float_as_uint(v0.w) != xi.id)
                             hit |= 1ull << (t - t0);
-                        if (two && dist2f(v1) < rl2f && __float_as_uint(v1.w) != xi.id)
+                        if (two && !(dist2f(v1) >= bd.hi) && __float_as_uint(v1.w) != xi.id)
                             hit |= 1ull << (t + LP - t0);
                     }
                     while (hit) {
@@ -2861,8 +2873,9 @@ __global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1) k_
                         hit &= hit - 1ull;
                         const int q = at(t0 + b);
                         const float4 v = lpos[q];
-                        bool far = !(dist2f(v) < rl2wf);
-                        if (exact) {
+                        const float d2 = dist2f(v);
+                        bool far = !(d2 < bd.wlo);
+                        if (!(d2 < bd.lo) || (far && !(d2 >= bd.whi))) {
                             const double r2 = dist2(a.X[lslot[q]]);
                             if (!(r2 < a.rl2))
                                 continue;
