@@ -9,6 +9,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <cmath>
 #include <stdint.h>
 
 namespace mdx {
@@ -381,6 +382,37 @@ __device__ __forceinline__ void bend_cosine(const R ab[3], const R bc[3], R k0, 
         R f3 = k0 * (ab[j] * inv - c * bc[j] / mbcsq);
         out[j] = role == 0 ? f1 : (role == 2 ? f3 : -(f1 + f3));
     }
+}
+
+// ----------------------------------------------------- form of the list build
+constexpr int NB_CAP_S = 800;   // staged particles per z offset (sparse)
+constexpr int NB_CAP_D = 1152;  // (dense)
+constexpr int NB_ROWCAP = 1152; // staged cell offsets per z offset
+
+// The form of k_nbuild for n particles, per_row of them in an x-row of cells
+// (forced: 0 the smaller, 1 the larger staging, -1 by size).  Four lanes per
+// position while the longest lane bounds the build (us per step with 4 / 1 lanes,
+// tetrahedral and condensate, mixed: 4,000 particles 21.7 / 24.0 and 20.5 / 23.1,
+// 70,000 47.9 / 50.1 and 36.5 / 38.0, 130,000 55.1 / 54.7 and 43.5 / 42.6) and
+// the rows about a block's 64 positions can be staged at all: of a position's
+// lanes only one walks global memory (90,000 in rows of 351: 48.0 / 46.3).  The
+// larger staging where the smaller would not hold those rows (20,000 in rows of
+// 247: 30.5 / 30.3, 40,000 in rows of 236: 46.9 / 46.2 with the smaller / larger).
+struct NbForm {
+    int lanes; // per position
+    int dense; // NB_CAP_D
+};
+inline NbForm nbuild_form(long long n, double per_row, int forced)
+{
+    // what a block of that many positions stages per z offset: its rows and the
+    // rows about them (nine tenths of the room, as rows differ in their particles)
+    auto fits = [&](double positions, int cap) {
+        return !(per_row > 0) || (std::ceil(positions / per_row) + 3) * per_row <= 0.9 * cap;
+    };
+    NbForm f;
+    f.lanes = n <= 100000 && fits(64, NB_CAP_D) ? 4 : 1;
+    f.dense = forced >= 0 ? forced != 0 : !fits(256 / f.lanes, NB_CAP_S);
+    return f;
 }
 
 } // namespace mdx

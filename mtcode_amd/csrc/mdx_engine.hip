@@ -1097,8 +1097,6 @@ template <class R> static int build_list(mdx_engine *e, const int *cells, int ga
 {
     KArgs<R> a = make_args<R>(e);
     a.lmode = 1;
-    // the larger LDS staging where an x-row of cells holds many particles
-    // (about 3 + 256 / row rows of particles staged per z offset of a block)
     long long rows = 0;
     double lmax = 0;
     for (const DevRep &r : e->reps) {
@@ -1106,10 +1104,6 @@ template <class R> static int build_list(mdx_engine *e, const int *cells, int ga
         lmax = std::max(lmax, std::max(r.l[0], std::max(r.l[1], r.l[2])));
     }
     const double per_row = rows > 0 ? (double)e->N / (double)rows : 0.0;
-    const bool dense =
-        e->nb_dense >= 0
-            ? e->nb_dense != 0
-            : per_row > 0 && (std::ceil(256.0 / per_row) + 3.0) * per_row > 0.9 * NB_CAP_S;
     // FP32 distances of coordinates within twice the box edge L, against a list
     // radius rl: a component is off by at most 6 * 2^-24 (L + rl) (two
     // coordinates by 2 each, the edge and the difference by 1), less than E, so
@@ -1122,13 +1116,12 @@ template <class R> static int build_list(mdx_engine *e, const int *cells, int ga
 #define NBUILD(CAP, LP)                                                                          \
     hipLaunchKernelGGL((k_nbuild<R, CAP, LP>), dim3(nblk(e->N, 256 / LP)), blk, 0, e->stream, a,  \
                        cells, gated, bd)
-    // four lanes per position while the longest lane bounds the build (us per
-    // step with 4 / 1 lanes, tetrahedral and condensate, mixed: 4,000 particles
-    // 21.7 / 24.0 and 20.5 / 23.1, 70,000 47.9 / 50.1 and 36.5 / 38.0, 130,000
-    // 55.1 / 54.7 and 43.5 / 42.6)
-    if (e->N <= 100000)
+    const NbForm form = nbuild_form(e->N, per_row, e->nb_dense);
+    if (form.lanes == 4 && form.dense)
+        NBUILD(NB_CAP_D, 4);
+    else if (form.lanes == 4)
         NBUILD(NB_CAP_S, 4);
-    else if (dense)
+    else if (form.dense)
         NBUILD(NB_CAP_D, 1);
     else
         NBUILD(NB_CAP_S, 1);

@@ -2468,6 +2468,11 @@ __global__ void __launch_bounds__(256) k_integrate(KArgs<R> a)
         drift_bound(a, drift);
 }
 
+// k_upkeep: ticket counter, then done counts per phase, each in a line of its
+// own (the waiting blocks' reads would hold up the others)
+constexpr int UP_LINE = 32, UP_SYNC = 3 * UP_LINE;
+constexpr int UP_BUCKET = 4;   // k_upkeep: arrivals per cell held in its bucket
+
 // neighbour list of every particle from the cell list of the current
 // positions: the slots within sqrt(rl2) in the order of a 27-cell walk
 // (z rows -1, 0, +1 outer, y rows -1, 0, +1 inner, then the cells x - 1,
@@ -2490,20 +2495,13 @@ __global__ void __launch_bounds__(256) k_integrate(KArgs<R> a)
 // within that bound of a radius is decided by its FP64 distance (NbBand), so the
 // list is the set of pairs within the radii in FP64 (mdx_list_pairs).
 // With FP64 records staged (32 B, two LDS reads per candidate, 38 KB) the walk
-// was bound by LDS reads and by 4 blocks per CU.  A block whose particles span more than NB_W rows or two
-// replicas, a grid with fewer than 3 cells on a side, and a z offset whose
-// rows hold more than NB_CAP particles or NB_ROWCAP cell offsets walk global
-// memory instead.  NB_CAP: 800 (26 KB of LDS, 6 blocks per CU) for sparse
-// systems, 1152 (33 KB, 4 blocks) where an x-row of cells holds many
-// particles (the host picks it from the mean particles per row).
-// k_upkeep: ticket counter, then done counts per phase, each in a line of its
-// own (the waiting blocks' reads would hold up the others)
-constexpr int UP_LINE = 32, UP_SYNC = 3 * UP_LINE;
-constexpr int UP_BUCKET = 4;   // k_upkeep: arrivals per cell held in its bucket
-constexpr int NB_W = 16;        // own x-rows of a block walked from LDS
-constexpr int NB_CAP_S = 800;   // staged particles per z offset (sparse)
-constexpr int NB_CAP_D = 1152;  // (dense)
-constexpr int NB_ROWCAP = 1152; // staged cell offsets per z offset
+// was bound by LDS reads and by 4 blocks per CU.  A block whose particles span
+// more than NB_W rows or two replicas, a grid with fewer than 3 cells on a side,
+// and a z offset whose rows hold more than NB_CAP particles or NB_ROWCAP cell
+// offsets walk global memory instead.  NB_CAP: 800 (26 KB of LDS, 6 blocks per
+// CU) for sparse systems, 1152 (33 KB, 4 blocks) where an x-row of cells holds
+// many particles; nbuild_form picks it and the lanes per position.
+constexpr int NB_W = 16; // own x-rows of a block walked from LDS
 
 // the list ranges [r0, r1) and [r2, r3) of the cells x - 1, x, x + 1 about
 // x-cell cx, in that order, in a row whose cell offsets are off[0..n0]

@@ -33,11 +33,10 @@ COPY_BYTES = 256 << 20
 # the phase each belongs to
 PHASES = {
     "bins": ("k_upkeep<float, 1>", "k_upkeep<float, 2>", "k_nbuild<float, 800, 1>",
-             "k_nbuild<float, 800, 4>", "k_nbuild<float, 1152, 1>"),
+             "k_nbuild<float, 800, 4>", "k_nbuild<float, 1152, 1>", "k_nbuild<float, 1152, 4>"),
     "walk": ("k_walkc<float, 3, false>",),
     "patch": ("k_patch<float, 3, false>", "k_patch_ovf<float, 3>"),
-    "finish": ("k_integrate<float, 3>", "k_integrate<float, 3, false>",
-               "k_integrate<float, 3, true>"),
+    "finish": ("k_integrate<float, 3, false>", "k_integrate<float, 3, true>"),
 }
 
 
