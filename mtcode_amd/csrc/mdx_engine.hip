@@ -2191,25 +2191,18 @@ int mdx_pair_histogram(mdx_engine *e, int replica, double max, double dx, long l
             return set_err(MDX_ERR_ARG, "max larger than the box");
     }
     int rc;
-    // edge[b]: the smallest squared distance in bin b or a later one, with the
-    // reference's floor(sqrt(d2) / dx)
-    auto bin_of = [&](double d2) { return std::floor(std::sqrt(d2) / dx); };
-    std::vector<double> edge((size_t)gs + 1, 0.0);
-    for (int k = 1; k <= gs; k++) {
-        double d2 = (k * dx) * (k * dx);
-        while (bin_of(d2) >= k)
-            d2 = std::nextafter(d2, 0.0);
-        while (bin_of(d2) < k)
-            d2 = std::nextafter(d2, HUGE_VAL);
-        edge[(size_t)k] = d2;
-    }
     if ((rc = custom_cells(e, replica, n)) ||
         (rc = dalloc(e, e->tmpll, 8 * (size_t)std::max(gs, 1))) ||
-        (rc = upload(e, e->aedge, edge.data(), edge.size())))
+        (rc = dalloc(e, e->aedge, 8 * ((size_t)gs + 1))))
         return rc;
     HIPCHK(hipMemsetAsync(e->tmpll.p, 0, 8 * (size_t)std::max(gs, 1), e->stream));
     const int cnt = e->nper[replica];
-    hipLaunchKernelGGL(k_gcount, dim3(nblk(cnt), 3), dim3(256), 8 * (size_t)(gs + 1) + 4 * (size_t)gs,
+    hipLaunchKernelGGL(k_gedges, dim3(nblk(gs + 1)), dim3(256), 0, e->stream, dx, gs,
+                       (double *)e->aedge.p);
+    // runs of 64 or more particles in parts while there are few blocks
+    const double run = 3.0 * cnt / ((double)n[0] * n[1] * n[2]);
+    const int parts = run < 64 ? 1 : std::min(8, std::max(1, 1024 / (3 * (int)nblk(cnt))));
+    hipLaunchKernelGGL(k_gcount, dim3(nblk(cnt), 3 * parts), dim3(256), 8 * (size_t)(gs + 1) + 4 * (size_t)gs,
                        e->stream, (const PosRec *)e->asorted.p, cnt, b[0], b[1], b[2], e->periodic,
                        n[0], n[1], n[2], (const int *)e->tmpi3.p, (const double *)e->aedge.p,
                        (float)(1.0 / dx), gs, (unsigned long long *)e->tmpll.p);

@@ -3649,10 +3649,12 @@ __global__ void __launch_bounds__(256) k_order_custom(int count, const int *cell
 // fn(record) for every particle after position q of the cell order in the
 // stencil's rows of z offset oz about cell c (the rows of k_pairs: -1, 0, 1
 // with 3 or more cells a side, 0, 1 with 2, 0 with 1).  The stencil is
-// symmetric, so over all q and oz each unordered pair comes up once.
+// symmetric, so over all q and oz each unordered pair comes up once.  (part of
+// parts: every parts-th of a run of particles, from its part-th)
 template <class Fn>
 __device__ __forceinline__ void for_each_after(const PosRec *sorted, const int *cstart, int q, int c,
-                                               int n0, int n1, int n2, int oz, Fn &&fn)
+                                               int n0, int n1, int n2, int oz, int part, int parts,
+                                               Fn &&fn)
 {
     const int cx = c % n0, cy = (c / n0) % n1, cz = c / (n0 * n1);
     if ((oz < 0 && n2 < 3) || (oz > 0 && n2 < 2))
@@ -3664,9 +3666,9 @@ __device__ __forceinline__ void for_each_after(const PosRec *sorted, const int *
         y = y < 0 ? y + n1 : (y >= n1 ? y - n1 : y);
         int r0, r1, r2, r3;
         row_ranges(cstart + n0 * (y + n1 * z), n0, cx, r0, r1, r2, r3);
-        for (int k = max(r0, q + 1); k < r1; k++)
+        for (int k = max(r0, q + 1) + part; k < r1; k += parts)
             fn(sorted[k]);
-        for (int k = max(r2, q + 1); k < r3; k++)
+        for (int k = max(r2, q + 1) + part; k < r3; k += parts)
             fn(sorted[k]);
     }
 }
@@ -3832,7 +3834,7 @@ __global__ void __launch_bounds__(256) k_cc_pairs(const PosRec *sorted, int coun
     if (some && k >= ex_lo && k <= ex_hi)
         return;
     const double l[3] = {l0, l1, l2};
-    for_each_after(sorted, cstart, q, (int)xi.meta, n0, n1, n2, (int)blockIdx.y - 1,
+    for_each_after(sorted, cstart, q, (int)xi.meta, n0, n1, n2, (int)blockIdx.y - 1, 0, 1,
                    [&](const PosRec &xj) {
                        const int j = (int)xj.id;
                        if (dlt(&xi.x, &xj.x, l, periodic, cut) && !(some && j >= ex_lo && j <= ex_hi))
@@ -3858,12 +3860,31 @@ __global__ void k_cc_flatten(int *lab, int n)
 // (geometry.h:107-123), bin floor(dis / dx) counted when below gs.  Counts are
 // integers: the order of the pairs does not change them.  sqrt, the division
 // and floor are monotonic, so a bin is a range of squared distances: edge[b]
-// is the smallest double whose bin is b or more (found on the host with the
-// same operations), and a pair takes an FP32 guess and comparisons in place of
+// is the smallest double whose bin is b or more (k_gedges), and a pair takes an FP32 guess and comparisons in place of
 // an FP64 root and division.  Bound by those FP64 operations and by scattered
 // reads before (one thread per particle in index order, every pair's root:
 // 381 us for 100,003 particles, 45 million pairs, 4.0 / 0.05).
+// blockIdx.y: z offset, then part of each run of particles (the host's number of
+// parts: several where a few blocks would search crowded cells).
 constexpr int GMAXB = 4096;
+
+// edge[b], with the pair's own operations.  (b dx)^2 is within a few roundings
+// of it, so both walks are a few steps (on the host 110 us for 4,096 bins)
+__global__ void __launch_bounds__(256) k_gedges(double dx, int gs, double *edge)
+{
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b > gs)
+        return;
+    auto bin_of = [&](long long bits) { return floor(sqrt(__longlong_as_double(bits)) / dx); };
+    // (doubles >= 0 are ordered as their bits)
+    long long d2 = __double_as_longlong((b * dx) * (b * dx));
+    while (d2 > 0 && bin_of(d2) >= b)
+        d2--;
+    while (bin_of(d2) < b)
+        d2++;
+    edge[b] = __longlong_as_double(d2);
+}
+
 __global__ void __launch_bounds__(256) k_gcount(const PosRec *sorted, int count, double l0,
                                                 double l1, double l2, int periodic, int n0, int n1,
                                                 int n2, const int *cstart, const double *edge,
@@ -3880,8 +3901,8 @@ __global__ void __launch_bounds__(256) k_gcount(const PosRec *sorted, int count,
     if (q < count && gs > 0) {
         const PosRec xi = sorted[q];
         const double end = sedge[gs];
-        for_each_after(sorted, cstart, q, (int)xi.meta, n0, n1, n2, (int)blockIdx.y - 1,
-                       [&](const PosRec &xj) {
+        for_each_after(sorted, cstart, q, (int)xi.meta, n0, n1, n2, (int)blockIdx.y % 3 - 1,
+                       (int)blockIdx.y / 3, (int)gridDim.y / 3, [&](const PosRec &xj) {
                            double temp = 0.0;
                            const double d[3] = {xi.x - xj.x, xi.y - xj.y, xi.z - xj.z};
                            const double l[3] = {l0, l1, l2};
@@ -3893,7 +3914,8 @@ __global__ void __launch_bounds__(256) k_gcount(const PosRec *sorted, int count,
                            }
                            if (!(temp < end))
                                return;
-                           int b = min((int)(sqrtf((float)temp) * inv_dx), gs - 1);
+                           // (0 times an infinite inv_dx: the last bin)
+                           int b = (int)fminf(sqrtf((float)temp) * inv_dx, (float)(gs - 1));
                            while (temp < sedge[b])
                                b--;
                            while (temp >= sedge[b + 1])
