@@ -634,6 +634,29 @@ __device__ __forceinline__ uint32_t cone_mask(const ScreenTab &tb, int ty, const
     return m;
 }
 
+// the same mask for a particle of a pair about to be evaluated, in the engine's
+// own precision (FP64: from the FP64 directions, 1e-12 below cos(theta_m))
+template <class R>
+__device__ __forceinline__ uint32_t pair_mask(const KArgs<R> &a, const PatchTab &tb, int ty,
+                                              const R q[9], const double u[3], const float uf[3],
+                                              float sign)
+{
+    if constexpr (sizeof(R) == 4) {
+        return cone_mask(tb, ty, q, uf, sign, (float)a.costm_screen_f);
+    } else {
+        const double v[3] = {q[0] * u[0] + q[1] * u[1] + q[2] * u[2],
+                             q[3] * u[0] + q[4] * u[1] + q[5] * u[2],
+                             q[6] * u[0] + q[7] * u[1] + q[8] * u[2]};
+        const double *d = tb.dird + 3 * tb.pstart[ty];
+        const int np = tb.np[ty];
+        uint32_t m = 0;
+        for (int k = 0; k < np; k++, d += 3)
+            m |= ((double)sign * (d[0] * v[0] + d[1] * v[1] + d[2] * v[2]) > a.costm_screen ? 1u : 0u)
+                 << k;
+        return m;
+    }
+}
+
 // roles of a patch pair: "a" = lower original index, exchanged when its type
 // is higher (GeneralPatch rows exist for ta <= tc; the potential is symmetric)
 __device__ __forceinline__ bool patch_roles(uint32_t oi, int ti, uint32_t oj, int tj, int &ta,
@@ -679,18 +702,10 @@ __device__ __forceinline__ int patch_pair(const KArgs<R> &a, const PatchTab &tb,
     // the screens; the decisions are then taken on the reference's own FP64
     // expressions
     const float uf[3] = {(float)u[0], (float)u[1], (float)u[2]};
-    float qs[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++)
-        qs[k] = (float)qa[k];
-    const float scr = (float)a.costm_screen_f;
-    const uint32_t ma = cone_mask(tb, ta, qs, uf, -1.f, scr);
+    const uint32_t ma = pair_mask(a, tb, ta, qa, u, uf, -1.f);
     if (!ma)
         return 0;
-#pragma unroll
-    for (int k = 0; k < 9; k++)
-        qs[k] = (float)qc[k];
-    const uint32_t mc = cone_mask(tb, tc, qs, uf, 1.f, scr);
+    const uint32_t mc = pair_mask(a, tb, tc, qc, u, uf, 1.f);
     const int npc = tb.np[tc];
     const double *da = tb.dird + 3 * tb.pstart[ta];
     const double *dc = tb.dird + 3 * tb.pstart[tc];
@@ -3971,18 +3986,10 @@ __global__ void __launch_bounds__(256) k_patch_bonds(KArgs<R> a, int *bonds)
             const R *qc = i_is_a ? qj : qi;
             // the cone screens of both sides first, as in patch_pair
             const float uf[3] = {(float)u[0], (float)u[1], (float)u[2]};
-            const float scr = (float)a.costm_screen_f;
-            float qf[9];
-#pragma unroll
-            for (int k = 0; k < 9; k++)
-                qf[k] = (float)qa[k];
-            const uint32_t ma = cone_mask(tb, ta, qf, uf, -1.f, scr);
+            const uint32_t ma = pair_mask(a, tb, ta, qa, u, uf, -1.f);
             if (!ma)
                 return;
-#pragma unroll
-            for (int k = 0; k < 9; k++)
-                qf[k] = (float)qc[k];
-            const uint32_t mc = cone_mask(tb, tc, qf, uf, 1.f, scr);
+            const uint32_t mc = pair_mask(a, tb, tc, qc, u, uf, 1.f);
             const int npc = tb.np[tc];
             const double *da = tb.dird + 3 * tb.pstart[ta];
             const double *dc = tb.dird + 3 * tb.pstart[tc];
