@@ -398,10 +398,6 @@ __device__ __forceinline__ bool face_clear(const KArgs<R> &a, const DevRep &rp, 
 }
 
 // ------------------------------------------------------------- gather kernel
-// the walk screens patch candidates (cone screens) before handing them over
-#ifndef MDX_WALK_SCREEN
-#define MDX_WALK_SCREEN 1
-#endif
 // neighbour-list entries loaded together per round of the list walk
 #ifndef MDX_LBATCH
 #define MDX_LBATCH 4
@@ -922,8 +918,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, const PatchT
         return (a.active_mask >> (ta * MAXT + tc)) & 1ull;
     };
     // the candidates the split form hands over: those that pass the screen
-    auto is_listed_candidate = [&](const PosRec &xj, int js, const double d[3], double r2s) -> bool {
-        (void)js;
+    auto is_listed_candidate = [&](const PosRec &xj, const double d[3], double r2s) -> bool {
         return is_patch_candidate(xj, r2s) && own_screen(a, *tb, ti, qs, d, r2s);
     };
     if (PH == PH_FINISH) {
@@ -940,8 +935,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, const PatchT
                 min_image(a, rp, xi.x, xi.y, xi.z, xj, d);
                 const double r2s = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
                 const int js = j >= 0 ? j : a.slot[xj.id];
-                if (!(r2s < a.rmax2) ||
-                    !(MDX_WALK_SCREEN ? is_listed_candidate(xj, js, d, r2s) : is_patch_candidate(xj, r2s)))
+                if (!(r2s < a.rmax2) || !is_listed_candidate(xj, d, r2s))
                     return;
                 if (seen++ >= a.pcap)
                     patch_pair<R, MODE>(a, *tb, rp, xi, ti, qi, js, acc);
@@ -982,7 +976,7 @@ __device__ __forceinline__ void process_particle(const KArgs<R> &a, const PatchT
             wca_term<R, MODE>(a, d, r2s, xj.id, exc0, exc1, acc);
             if (PH == PH_WALK) {
                 const int js = j >= 0 ? j : a.slot[xj.id];
-                if (MDX_WALK_SCREEN ? is_listed_candidate(xj, js, d, r2s) : is_patch_candidate(xj, r2s)) {
+                if (is_listed_candidate(xj, d, r2s)) {
                     if (npc < a.pcap)
                         a.cand[(size_t)npc * a.N + s] = js;
                     npc++;
@@ -2277,7 +2271,7 @@ __device__ __forceinline__ void patch_overflow(const KArgs<R> &a, const PatchTab
         patch_roles(xi.id, ti, xj.id, tj, ta, tc);
         if (!((a.active_mask >> (ta * MAXT + tc)) & 1ull))
             return;
-        if (MDX_WALK_SCREEN && !own_screen(a, tb, ti, qs, d, r2s))
+        if (!own_screen(a, tb, ti, qs, d, r2s))
             return;
         const int js = j >= 0 ? j : a.slot[xj.id];
         if (seen++ >= a.pcap)
