@@ -433,8 +433,9 @@ static int fetch(mdx_engine *e, const Span *sp, int n, bool joined, W &&meanwhil
     try {
         for (; started < FETCH_THREADS; started++)
             th[started] = std::thread(work);
-    } catch (const std::system_error &) {
-        // fewer threads; none: this one empties the slots too
+    } catch (...) {
+        // fewer threads (no more of them, or no memory for one); none: this one
+        // empties the slots too
     }
     for (size_t c = 0; c < pieces && he == hipSuccess; c++) {
         // the slots whose pieces have been emptied take the next pieces; piece c
