@@ -36,7 +36,9 @@ PHASES = {
              "k_nbuild<float, 800, 4>", "k_nbuild<float, 1152, 1>", "k_nbuild<float, 1152, 4>"),
     "walk": ("k_walkc<float, 3, false>",),
     "patch": ("k_patch<float, 3, false>", "k_patch_ovf<float, 3>"),
-    "finish": ("k_integrate<float, 3, false>", "k_integrate<float, 3, true>"),
+    # (the form without the topology switch: summaries of older profiles)
+    "finish": ("k_integrate<float, 3>", "k_integrate<float, 3, false>",
+               "k_integrate<float, 3, true>"),
 }
 
 

@@ -108,3 +108,21 @@ def test_long_boxes(n, box, periodic, kind):
     want = _within(s, tree.query_pairs(rl * (1 + 1e-6), output_type="ndarray"), rl, rw)
     assert len(want) > 300
     assert np.array_equal(got, _sorted(want))
+
+
+@pytest.mark.parametrize("kind", ["tetra", "condensate"])
+@pytest.mark.parametrize("forced", ["", "0", "1"])
+@pytest.mark.parametrize("n,box", [(63, (9.0, 9.0, 9.0)), (65, (30.0, 7.0, 7.0)),
+                                   (6000, (300.0, 11.0, 11.0)),  # 240 particles in a row of cells
+                                   (8750, (400.0, 11.0, 11.0)),  # 350
+                                   (5000, (24.0, 24.0, 24.0))])
+def test_forms_of_the_build(n, box, forced, kind, monkeypatch):
+    """both stagings, by size and forced, and rows that neither holds"""
+    if forced:
+        monkeypatch.setenv("MDX_NBDENSE", forced)
+    box = np.array(box)
+    s = _system(n, box, np.random.default_rng(n).uniform(0, 1, (n, 3)) * box, kind, True)
+    got, rl, rw = _list(s)
+    tree = cKDTree(s["x"], boxsize=box)
+    want = _within(s, tree.query_pairs(rl * (1 + 1e-6), output_type="ndarray"), rl, rw)
+    assert np.array_equal(got, _sorted(want))
