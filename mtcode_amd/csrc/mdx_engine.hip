@@ -739,6 +739,17 @@ template <class R> static int count_current(mdx_engine *e)
     return MDX_OK;
 }
 
+// The positions change and the counts taken of them will not be scanned (a bead
+// step without the list counts the positions it writes): cleared, since the next
+// binning adds to what is there.
+static int drop_counts(mdx_engine *e)
+{
+    if (e->counted)
+        HIPCHK(hipMemsetAsync(e->count.p, 0, sizeof(int) * ((size_t)e->ncells + 1), e->stream));
+    e->counted = false;
+    return MDX_OK;
+}
+
 // cell list of the current slots (no reordering)
 template <class R> static int bin_current(mdx_engine *e)
 {
@@ -1639,9 +1650,8 @@ static int upload_state_t(mdx_engine *e, const double *x, const double *p, const
     e->cur = 0;
     e->binned = false;
     e->primed = false;
-    e->counted = false;
     e->list_valid = false;
-    return MDX_OK;
+    return drop_counts(e);
 }
 
 int mdx_upload_state(mdx_engine *e, const double *x, const double *p, const double *Q,
@@ -3114,14 +3124,14 @@ int mdx_info(mdx_engine *e, double *out)
 // Each changes the engine's state in place (slot order kept); afterwards the
 // carried forces of mdx_step are stale (mdx_prime again) and, if positions
 // moved, so are the cell and neighbour lists.
-static void stage_done(mdx_engine *e, bool moved)
+static int stage_done(mdx_engine *e, bool moved)
 {
     e->primed = false;
-    if (moved) {
-        e->binned = false;
-        e->counted = false;
-        e->list_valid = false;
-    }
+    if (!moved)
+        return MDX_OK;
+    e->binned = false;
+    e->list_valid = false;
+    return drop_counts(e);
 }
 
 // up to three host arrays (n[k] doubles) into device buffers: through the
@@ -3169,8 +3179,7 @@ template <class R> static int stage_halfkick_t(mdx_engine *e, const double *F, c
                        rot ? (const double *)e->tmpx.p : nullptr, e->dt / 2.);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
-    stage_done(e, false);
-    return MDX_OK;
+    return stage_done(e, false);
 }
 
 int mdx_stage_halfkick(mdx_engine *e, const double *F, const double *T)
@@ -3191,7 +3200,8 @@ template <class R> static int stage_advance_pos_t(mdx_engine *e)
                        (PosRec *)e->X[e->cur].p, (R *)e->P[e->cur].p, (const DevRep *)e->dreps.p,
                        e->dt / e->m, e->periodic, (StepCtl *)e->ctl.p);
     HIPCHK(hipGetLastError());
-    stage_done(e, true);
+    if ((rc = stage_done(e, true)))
+        return rc;
     unsigned int st;
     if ((rc = read_status(e, &st)))
         return rc;
@@ -3212,8 +3222,7 @@ template <class R> static int stage_rotate_t(mdx_engine *e)
                        (R *)e->Lm[e->cur].p, (R *)e->Q[e->cur].p, e->dt, e->I[0], e->I[1], e->I[2]);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
-    stage_done(e, false);
-    return MDX_OK;
+    return stage_done(e, false);
 }
 
 int mdx_stage_rotate(mdx_engine *e)
@@ -3247,8 +3256,7 @@ template <class R> static int stage_sphere_t(mdx_engine *e, double *F, double *T
     const Span out[2] = {{F, e->tmpd.p, 8 * n3}, {T, e->tmpx.p, 8 * n3}};
     if ((rc = fetch(e, out, 2)))
         return rc;
-    stage_done(e, false);
-    return MDX_OK;
+    return stage_done(e, false);
 }
 
 int mdx_stage_sphere(mdx_engine *e, double *F, double *T, const double *RT)
@@ -3281,8 +3289,7 @@ template <class R> static int stage_advance_mom_t(mdx_engine *e, const double *F
                        (const double *)e->tmpx.p, c5 * c2, (c5 * (c3) + q), c2, c5);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
-    stage_done(e, false);
-    return MDX_OK;
+    return stage_done(e, false);
 }
 
 int mdx_stage_advance_mom(mdx_engine *e, const double *F, const double *R)
