@@ -1,13 +1,18 @@
 // mdx_engine.hip -- MI355X (gfx950) engine behind include/mdx.h (host side).
 //
-// Per step (rotor integrator, Condensate.cpp:352-377 of the reference):
-//   exclusive scan of cell counts -> fill cell lists -> order each cell's list
-//   -> gather forces + sphere + half kick (+ the next step's half kick, drift,
-//      rotation and binning, fused)
-// The gather kernel (mdx_kernels.h) computes every particle's force and torque
-// by looping over its 27 neighbour cells (full neighbour list, no Newton-3
-// scatter, no atomics), so results are deterministic, and re-sorts the state
-// into cell order as it writes the next step.
+// Per step (rotor integrator, Condensate.cpp:352-377 of the reference), with the
+// neighbour list (the default):
+//   k_upkeep (displacement bound; when it is used up, the cell list of the
+//   current slots) -> k_nbuild (then the new neighbour list) -> forces, sphere
+//   step, both half kicks, drift and rotation: k_cstep for small systems, else
+//   k_walkc -> k_patch -> k_integrate, or the fused form of the first two
+// Without the list, for single steps and every resort_every steps: scan of the
+// cell counts -> cell lists -> their order -> forces from the 27 cells about
+// each particle (k_cgather, k_gather, or k_walk and the patch kernels), with the
+// next step's half kick, drift, rotation and binning; the state is re-sorted
+// into cell order as it is written.
+// Every particle's force and torque is summed over its own neighbours (no
+// Newton-3 scatter, no atomics), so results are deterministic.
 //
 // Reference paths in comments are relative to the reference's Code/ folder.
 #include "mdx_kernels.h"
@@ -26,7 +31,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>

@@ -1,12 +1,12 @@
 // mdx_kernels.h -- gfx950 kernels of the Langevin step.
 //
-// Storage order.  Particles live in "slots".  Every kernel that produces the
-// next state is launched with one thread per slot of the *cell list* order:
-// thread s takes the particle in old slot list[s], and writes its next state
-// to slot s of the other buffer.  The state is therefore re-sorted into cell
-// order every step without an extra pass, so that the threads of a wavefront
-// handle particles of the same or adjacent cells (shared neighbour cells,
-// coalesced gathers).  Each particle carries its original index (id): noise
+// Storage order.  Particles live in "slots".  A step from the cells takes the
+// positions of the *cell list* in order: position s is the particle in old slot
+// list[s], and its next state goes to slot s of the other buffer.  The state is
+// therefore re-sorted into cell order without an extra pass, so that the threads
+// of a wavefront handle particles of the same or adjacent cells (shared
+// neighbour cells, coalesced gathers).  Steps that walk the neighbour list keep
+// the slots.  Each particle carries its original index (id): noise
 // counters, the p1 < p2 roles of the patch loop, topology and the host
 // interface all use it.
 //
