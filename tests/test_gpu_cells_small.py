@@ -18,7 +18,7 @@ BOXES = pytest.mark.parametrize("n,box,cells", [
 @BOTH
 @BOXES
 def test_few_cells_a_side(n, box, cells, precision, monkeypatch):
-    s = _fluid(n, box=np.array(box))
+    s = _fluid(n, box=box)
     with mdx.engine_from_system(s, precision=precision) as e:
         assert e.info()["cells"] == cells[0] * cells[1] * cells[2]
     _same(s, precision, monkeypatch)
@@ -26,7 +26,7 @@ def test_few_cells_a_side(n, box, cells, precision, monkeypatch):
 
 @BOXES
 def test_wca_of_every_pair(n, box, cells):
-    s = _fluid(n, box=np.array(box))
+    s = _fluid(n, box=box)
     s["wca"] = (1.0, 1.0, 0.0)
     s["patches"]["params"][:, 0] = 1e-300  # the patch path, without its forces
     with mdx.engine_from_system(s, precision=mdx.PREC_FP64) as e:
