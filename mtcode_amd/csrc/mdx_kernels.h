@@ -2725,10 +2725,11 @@ __global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1)
             hf[k] = a.periodic ? 0.5f * lf[k] : 3.0e38f;
         }
         // (NaN beyond twice the edge, where the bands do not hold: the FP64
-        // distance decides every candidate of such a particle)
+        // distance decides every candidate of such a particle.  From the table
+        // and not lf, which would spill: 2 registers, 2 us of a 110 us rebuild)
         auto coarse = [&](double x, int k) -> float {
             const float v = (float)x;
-            return fabsf(v) <= 2.f * lf[k] ? v : __uint_as_float(0x7fc00000u);
+            return fabsf(v) <= 2.f * (float)rb.l[k] ? v : __uint_as_float(0x7fc00000u);
         };
         const float xf[3] = {coarse(xi.x, 0), coarse(xi.y, 1), coarse(xi.z, 2)};
         const int wv = tid >> 6, lane = tid & 63;
