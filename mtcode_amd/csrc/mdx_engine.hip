@@ -1493,7 +1493,10 @@ int mdx_create(const mdx_desc *d, mdx_engine **out)
     // the one-kernel form while its blocks are all resident: FP64 us per step
     // (tetrahedral / condensate) 54.7 / 44.8 against 58.7 / 44.7 split at
     // 32,000 particles, 82 / 62 against 60 / 47 at 50,000; mixed 39 / 33
-    // against 56 / 42 at 32,000, 54.5 / 45.4 against 55.7 / 43.8 at 50,000
+    // against 56 / 42 at 32,000, 54.5 / 45.4 against 55.7 / 43.8 at 50,000.
+    // Beads (either precision) and polymers cross in between: beads 22.1 against
+    // 25.9 at 20,800, 27.3 / 26.7 at 41,600, 31.0 / 27.5 at 62,400; polymers 29.3
+    // / 37.0 at 25,600, 42.9 / 40.7 at 40,960
     const long long split_min = e->prec == MDX_PREC_FP64 ? 32768 : 45000;
     e->use_split = N > split_min;
     if (const char *t = std::getenv("MDX_TILES"))

@@ -2550,8 +2550,9 @@ struct NbBand {
 
 // The sparse one-lane form is held to 80 VGPRs (6 waves per SIMD, no spill: 120
 // -> 106 us).  Measured, a rebuild's list: 1,048,576-particle condensate 145
-// (FP64 records) -> 106 us, 64 replicas (298,897) 98 -> 76, 262,144 polymer
-// beads 68 -> 61, 4,096 particles 42 -> 19 (four lanes per position).
+// (FP64 records) -> 106 us (110 with the FP64 decision near the radii), 64
+// replicas (298,897) 98 -> 76, 262,144 polymer beads 68 -> 61, 4,096 particles
+// 42 -> 19 (four lanes per position).
 template <class R, int NB_CAP, int LP>
 __global__ void __launch_bounds__(256, LP == 1 && NB_CAP == NB_CAP_S ? 6 : 1)
     k_nbuild(KArgs<R> a, const int *cells, int gated, NbBand bd)
